@@ -55,6 +55,21 @@ constexpr int WS_CSLOT = WS_TB * 32;     // floats per cos (or sin) slot
 
 __device__ constexpr int swz(int r) { return (r >> 1) & 7; }
 
+// FP32 outputs (the residual and BIAS_F32 epilogues) run the MFMA with the
+// operands in the other order -- the same products, summed in the same order --
+// so that a lane holds one column and four tokens: adjacent lanes then store
+// adjacent columns, 64 bytes a token.  With four columns per lane, sixteen
+// tokens side by side, a 16-byte store or load ran at 37 B/ns per CU in a probe
+// on MI355X against 57 (stores) and 102 (loads) in runs of 64 bytes.  Measured
+// (us per launch, 9482 / 16384 / 131072 tokens): Wo 19.0 / 27.6 / 251 -> 18.4 /
+// 26.5 / 239, the K = 1152 kernel 23.4 / 47.5 / 338 -> 22.8 / 47.5 / 332.
+//
+// Residual rows of a 16-token x 16-column group reach LDS by one DMA
+// instruction, lane l bringing 16-byte chunk l % 4 of token old_token(l): tokens
+// 4kg + i lie at row 4i + kg of [16][16] floats, so that the 64 lanes of a
+// read (tokens 4kg + i of four kg, sixteen columns each) cover all banks.
+__device__ inline int old_token(int lane) { return 4 * ((lane >> 2) & 3) + (lane >> 4); }
+
 template <int EPI>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void gemm_ws_kernel(GemmArgs a, int nF,
                                                                                                int R, int nTB) {
@@ -74,9 +89,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
     __shared__ __align__(16) int spos[ROPE ? WS_NCS * 64 : 4];   // token metadata of a block, DMA'd
     constexpr bool RESID = EPI == JH_EPI_RESID_F32;
     __shared__ __align__(16) f32x4 sold[RESID ? 8 : 1][2][64];   // [wave][lo/hi][lane]: residual rows, by DMA
-    // [wave][lo/hi][lane]: the bias values of the lane's columns, by DMA in the prologue (a register load in
-    // the epilogue would wait, with vmcnt(0), for the X DMA issued before it)
-    __shared__ __align__(16) f32x4 sbias[BIASED || RESID ? 8 : 1][2][64];
+    // [wave][lo/hi][lane]: the bias values of the lane's columns (one per lane for the FP32 outputs), by DMA in
+    // the prologue (a register load in the epilogue would wait, with vmcnt(0), for the X DMA issued before it)
+    __shared__ __align__(16) f32x4 sbias[BIASED || RESID ? 8 : 1][2][F32OUT ? 16 : 64];
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -159,14 +174,19 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
         if (two) issue_pos(b0 + 1, 1);
         if constexpr (BIASED || RESID) {
             if (a.bias) {
-                const int bcol = 64 * (4 * f + (wave >> 1)) + 16 * (wave & 1) + 4 * (lane >> 4);
+                const int bcol = 64 * (4 * f + (wave >> 1)) + 16 * (wave & 1) + (F32OUT ? lane & 15 : 4 * (lane >> 4));
                 const i32x4 rb = make_rsrc(a.bias, (uint64_t)a.n * 4);
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     const uint32_t m0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)&sbias[wave][h][0]);
-                    asm volatile("buffer_load_dwordx4 %1, %2, %3 offen lds" ::"{m0}"(m0), "v"((uint32_t)bcol * 4),
-                                 "s"(rb), "s"(h * 128)
-                                 : "memory");
+                    if constexpr (F32OUT)
+                        asm volatile("buffer_load_dword %1, %2, %3 offen lds" ::"{m0}"(m0), "v"((uint32_t)bcol * 4),
+                                     "s"(rb), "s"(h * 128)
+                                     : "memory");
+                    else
+                        asm volatile("buffer_load_dwordx4 %1, %2, %3 offen lds" ::"{m0}"(m0), "v"((uint32_t)bcol * 4),
+                                     "s"(rb), "s"(h * 128)
+                                     : "memory");
                 }
             }
         }
@@ -240,8 +260,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
         }
         if constexpr (BIASED) {
             if (j == 0) {
-                e.c = sbias[wave][0][lane];
-                e.sn = sbias[wave][1][lane];
+                if constexpr (F32OUT) {
+                    const float bl = ((const float*)sbias[wave][0])[lane], bh = ((const float*)sbias[wave][1])[lane];
+                    e.c = f32x4{bl, bl, bl, bl};
+                    e.sn = f32x4{bh, bh, bh, bh};
+                } else {
+                    e.c = sbias[wave][0][lane];
+                    e.sn = sbias[wave][1][lane];
+                }
             } else {
                 e.lo[j - 1] += e.c[j - 1];
                 e.hi[j - 1] += e.sn[j - 1];
@@ -271,28 +297,34 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
             __builtin_amdgcn_raw_buffer_store_b64(u32x2{pack2(e.lo[0], e.lo[1]), pack2(e.lo[2], e.lo[3])}, ro, vo,
                                                   0, 0);
         } else if constexpr (F32OUT) {
-            if constexpr (EPI == JH_EPI_RESID_F32) {
-                // the residual rows, DMA'd into LDS a block ahead (issue_old)
-                const f32x4 olo = sold[wave][0][lane], ohi = sold[wave][1][lane];
-                f32x4 lo = e.lo, hi = e.hi;
+            // Lane (tk, kg): column tk of each half, tokens 4kg .. +3.
+            float lo[4], hi[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                lo[i] = e.lo[i];
+                hi[i] = e.hi[i];
+            }
+            if constexpr (RESID) {
                 if (a.bias) {
-                    const f32x4 b_lo = sbias[wave][0][lane], b_hi = sbias[wave][1][lane];
+                    const float bl = ((const float*)sbias[wave][0])[lane], bh = ((const float*)sbias[wave][1])[lane];
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        lo[i] += b_lo[i];
-                        hi[i] += b_hi[i];
+                        lo[i] += bl;
+                        hi[i] += bh;
                     }
                 }
+                // the residual rows, DMA'd into LDS a block ahead (issue_old)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    lo[i] = olo[i] + lo[i];
-                    hi[i] = ohi[i] + hi[i];
+                    lo[i] = ((const float*)sold[wave][0])[(4 * i + kg) * 16 + tk] + lo[i];
+                    hi[i] = ((const float*)sold[wave][1])[(4 * i + kg) * 16 + tk] + hi[i];
                 }
-                __builtin_amdgcn_raw_buffer_store_b128(lo, ro, vo, 0, 0);
-                __builtin_amdgcn_raw_buffer_store_b128(hi, ro, vo + 32 * ESZ, 0, 0);
-            } else {
-                __builtin_amdgcn_raw_buffer_store_b128(e.lo, ro, vo, 0, 0);
-                __builtin_amdgcn_raw_buffer_store_b128(e.hi, ro, vo + 32 * ESZ, 0, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int ro4 = (int)((4 * kg + i) * a.ldo + a.col + 64 * hb + x0 + tk) * 4;
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, lo[i]), ro, ro4, 0, 0);
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, hi[i]), ro, ro4 + 128, 0, 0);
             }
         } else {
             __builtin_amdgcn_raw_buffer_store_b64(u32x2{pack2(e.lo[0], e.lo[1]), pack2(e.lo[2], e.lo[3])}, ro, vo, 0,
@@ -312,9 +344,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
     auto issue_old = [&](int bb) {
         if constexpr (RESID) {
             const int t0 = bb * WS_TB, nt = a.rows - t0 < WS_TB ? a.rows - t0 : WS_TB;
-            const int col = a.col + 64 * hb + x0 + 4 * kg;
             const i32x4 ro = make_rsrc((const float*)a.out + (long)t0 * a.ldo, (uint64_t)nt * a.ldo * 4);
-            const uint32_t vo = (uint32_t)(tk * a.ldo + col) * 4;
+            const uint32_t vo = (uint32_t)(old_token(lane) * a.ldo + a.col + 64 * hb + x0 + 4 * (lane & 3)) * 4;
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const uint32_t m0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)&sold[wave][h][0]);
@@ -355,7 +386,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const bf16x8 w = s < WS_SR ? wf[s < WS_SR ? s : 0][h] : wl[(s - WS_SR) & 1][h];
-                acc[P][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, bx[s % WS_PD], acc[P][h], 0, 0, 0);
+                acc[P][h] = F32OUT ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(bx[s % WS_PD], w, acc[P][h], 0, 0, 0)
+                                   : __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, bx[s % WS_PD], acc[P][h], 0, 0, 0);
             }
             __builtin_amdgcn_sched_barrier(0);
             if (s + WS_PD < WS_S) bx[s % WS_PD] = rd(s + WS_PD);
@@ -391,16 +423,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
     // Each block starts with a barrier (its X, RoPE rows and positions
     // landed; the slots of two blocks back are free), for which each wave
     // waits for its own DMA, but not for the stores of the epilogue it ran
-    // since: those are its last VMEM instructions, 2 of them (1 for GEGLU),
-    // issued whether or not their rows are past the last token; with RESID
-    // the two residual-row DMAs of issue_old follow them (and, in the first
-    // block, come alone).
+    // since: those are its last VMEM instructions, 2 of them (1 for GEGLU, 8
+    // for the FP32 outputs), issued whether or not their rows are past the
+    // last token; with RESID the two residual-row DMAs of issue_old follow
+    // them (and, in the first block, come alone).
     auto sync = [&](int k) {
         if constexpr (RESID) {
             if (k == 1) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
-            else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+            else asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
         } else {
             if (k == 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            else if constexpr (F32OUT) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
             else if constexpr (GEGLU) asm volatile("s_waitcnt vmcnt(1)" ::: "memory");
             else asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
         }
@@ -461,7 +494,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
     __shared__ __align__(1024) bf16_t sx[2 * W2_XSLOT];
     __shared__ __align__(16) f32x4 spart[2][4][2][64];  // [block parity][row group][lo/hi][lane]
     __shared__ __align__(16) f32x4 sold[4][2][64];      // [row group][lo/hi][lane]: residual rows, by DMA
-    __shared__ __align__(16) f32x4 sbias[4][2][64];     // [row group][lo/hi][lane]: bias, by DMA in the prologue
+    __shared__ __align__(16) float sbias[4][2][64];     // [row group][lo/hi][lane]: bias, by DMA in the prologue
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -502,11 +535,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
         for (int j = 0; j < 5; ++j) issue_x(rx, 0, j);
         if (a.bias && kh == 0) {
             const i32x4 rb = make_rsrc(a.bias, (uint64_t)a.n * 4);
-            const uint32_t bo = (uint32_t)(W2_ROWS * f + 32 * rg + 4 * (lane >> 4)) * 4;
+            const uint32_t bo = (uint32_t)(W2_ROWS * f + 32 * rg + (lane & 15)) * 4;
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const uint32_t m0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)&sbias[rg][h][0]);
-                asm volatile("buffer_load_dwordx4 %1, %2, %3 offen lds" ::"{m0}"(m0), "v"(bo), "s"(rb), "s"(h * 64)
+                asm volatile("buffer_load_dword %1, %2, %3 offen lds" ::"{m0}"(m0), "v"(bo), "s"(rb), "s"(h * 64)
                              : "memory");
             }
         }
@@ -526,7 +559,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
     __syncthreads();
 
     const int tk = lane & 15, kg = lane >> 4;
-    const int col = a.col + W2_ROWS * f + 32 * rg + 4 * kg;  // lo columns; hi = col + 16
+    const int col = a.col + W2_ROWS * f + 32 * rg;  // first of the lo columns; hi = col + 16
     f32x4 acc[2][2];                                          // [set][lo/hi]
 
     // The residual values a lower-half wave's lanes add to (block bb, its 16
@@ -538,7 +571,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
     auto issue_old = [&](int bb) {
         const int t0 = bb * WS_TB, nt = a.rows - t0 < WS_TB ? a.rows - t0 : WS_TB;
         const i32x4 ro = make_rsrc((const float*)a.out + (long)t0 * a.ldo, (uint64_t)nt * a.ldo * 4);
-        const uint32_t vo = (uint32_t)(tk * a.ldo + col) * 4;
+        const uint32_t vo = (uint32_t)(old_token(lane) * a.ldo + col + 4 * (lane & 3)) * 4;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const uint32_t m0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)&sold[rg][h][0]);
@@ -553,31 +586,30 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
     auto epilogue = [&](int P, int bb) {
         const int t0 = bb * WS_TB, nt = a.rows - t0 < WS_TB ? a.rows - t0 : WS_TB;
         const f32x4 plo = spart[(bb - b0) & 1][rg][0][lane], phi = spart[(bb - b0) & 1][rg][1][lane];
-        const f32x4 olo = sold[rg][0][lane], ohi = sold[rg][1][lane];
-        f32x4 lo, hi;
+        float lo[4], hi[4];  // column tk of each half, tokens 4kg .. +3
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             lo[i] = acc[P][0][i] + plo[i];
             hi[i] = acc[P][1][i] + phi[i];
         }
         if (a.bias) {
-            const f32x4 b_lo = sbias[rg][0][lane], b_hi = sbias[rg][1][lane];
+            const float bl = sbias[rg][0][lane], bh = sbias[rg][1][lane];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                lo[i] += b_lo[i];
-                hi[i] += b_hi[i];
+                lo[i] += bl;
+                hi[i] += bh;
             }
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            lo[i] = olo[i] + lo[i];
-            hi[i] = ohi[i] + hi[i];
         }
         const __amdgpu_buffer_rsrc_t ro =
             __builtin_amdgcn_make_buffer_rsrc((char*)a.out + (long)t0 * a.ldo * 4, 0, nt * a.ldo * 4, 0x00020000);
-        const int vo = (tk * a.ldo + col) * 4;
-        __builtin_amdgcn_raw_buffer_store_b128(lo, ro, vo, 0, 0);
-        __builtin_amdgcn_raw_buffer_store_b128(hi, ro, vo + 64, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            lo[i] = ((const float*)sold[rg][0])[(4 * i + kg) * 16 + tk] + lo[i];
+            hi[i] = ((const float*)sold[rg][1])[(4 * i + kg) * 16 + tk] + hi[i];
+            const int vo = (int)((4 * kg + i) * a.ldo + col + tk) * 4;
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, lo[i]), ro, vo, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, hi[i]), ro, vo + 64, 0, 0);
+        }
     };
 
     // One block bb into accumulator set P from X slot (bb - b0) % 2: the
@@ -606,7 +638,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int h = 0; h < 2; ++h)
-                acc[P][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[s][h], bx[s % W2_PD], acc[P][h], 0, 0, 0);
+                acc[P][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bx[s % W2_PD], wf[s][h], acc[P][h], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
             if (s + W2_PD < W2_SH) bx[s % W2_PD] = rd(s + W2_PD);
             if (s == 1 || s == 3 || s == 5 || s == 7 || s == 9) issue_x(rx, (k + 1) & 1, s >> 1);
@@ -632,13 +664,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
 
     // Each block starts with a barrier: its X landed (each wave waits for its
     // own DMA, but a lower-half wave not for its last VMEM instructions: the
-    // two stores of its epilogue, none in the first block, and the two
+    // eight stores of its epilogue, none in the first block, and the two
     // residual-row DMAs after them), the previous block's upper-half sums are
     // in LDS, and the slots of two blocks back are free.
     auto sync = [&](int k) {
         if (kh == 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         else if (k == 1) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
         __syncthreads();
     };
     block(C0{}, F{}, b0);
