@@ -188,7 +188,10 @@ typedef struct jh_attn_tile {
  * q/k/v bf16 with row strides ldq/ldkv; head h reads columns [64h, 64h+64)
  * of each; out bf16 row stride ldo.  `tiles` is a device array; work items
  * are dispatched in list order with heads varying fastest, so listing the
- * costliest tiles first (as the backend does) balances the CUs.
+ * costliest tiles first (as the backend does) balances the CUs.  Full
+ * attention with few work items (at most two per CU) over long rows splits
+ * each item's keys over two or four groups of waves, which adds a query's
+ * partial sums in another order.
  * Replaces attention_rope/attention_plain (src/cuda/kernels.cu:274-391); RoPE
  * is applied by the producing GEMM's ROPE epilogue instead of on every load.
  */
@@ -199,8 +202,10 @@ int jh_op_attention(const void* q, size_t ldq, const void* k, const void* v, siz
 /*
  * jh_op_attention with work items of up to 256 queries (tiles of nq <= 256):
  * eight waves per (tile, head), each staged K/V tile shared by twice the
- * queries.  The backend uses it for the global layers of sequences of 4096
- * tokens or more.  Same arithmetic per query as jh_op_attention.  No separate
+ * queries, or two 128-query workgroups per tile where those leave fewer CUs
+ * idle (and on window layers).  The backend uses it for the global layers of
+ * sequences of 4096 tokens or more.  Same arithmetic per query as
+ * jh_op_attention for the same number of workgroups.  No separate
  * counterpart in the reference (part of attention_rope/attention_plain,
  * src/cuda/kernels.cu:274-391).
  */

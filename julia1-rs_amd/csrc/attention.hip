@@ -71,18 +71,20 @@ __device__ constexpr int vswz(int r) { return ((r >> 1) & 1) << 2; }
 // eight-wave form stages two key tiles per barrier (four 16 KB K/V slots,
 // 64 KB: two workgroups per CU still fit), which halves the barriers each
 // wave meets (a further 1.8% at 4 x 8192).
-template <int NW, bool WIN>  // WIN: a window layer (a.window >= 0), whose tiles run one 32-key block per step
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(4))) void attention_kernel(AttnArgs a) {
+// KS > 1 splits the keys of a 128-query item over KS groups of four waves: a
+// stage holds KS key tiles, group g runs tile g of each, and at the end the
+// groups' running maxima, sums and outputs are merged through LDS in group order.
+template <int NW, bool WIN, int KS>  // WIN: a window layer (a.window >= 0), whose tiles run one 32-key block per step
+__device__ __forceinline__ void attend(const AttnArgs& a, const AttnTile& tile, const int head,
+                                       bf16_t (&smem)[2][NW / 2][KT * 64]) {
+    static_assert(KS == 1 || NW == 4 * KS, "key-split items have 128 queries");
     constexpr int SPB = NW / 4;           // key tiles staged per barrier
     constexpr int RPW = SPB * KT / NW;    // K/V rows each wave stages per barrier (8 per DMA instruction)
-    __shared__ __align__(1024) bf16_t sK[2 * SPB][KT * 64];
-    __shared__ __align__(1024) bf16_t sV[2 * SPB][KT * 64];
-
-    // One workgroup per (tile, head), heads varying fastest: callers list the
-    // costliest tiles first, so those are dispatched first, one per CU.
-    const int head = (int)(blockIdx.x % (unsigned)a.heads);
-    const AttnTile tile = a.tiles[blockIdx.x / (unsigned)a.heads];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    auto& sK = smem[0];
+    auto& sV = smem[1];
+    const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = KS > 1 ? wid & 3 : wid;  // query group of the wave
+    const int kgrp = KS > 1 ? wid >> 2 : 0;   // key group of the wave
     const int lq = lane & 31, g = lane >> 5;
 
     const bf16_t* kbase = a.k + (long)tile.kv_row * a.ldkv + head * 64;
@@ -127,7 +129,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(4))) vo
     uint32_t okb[RPW / 8], ovb[RPW / 8];
 #pragma unroll
     for (int j = 0; j < RPW / 8; ++j) {
-        const int row = RPW * wave + 8 * j + (lane >> 3);
+        const int row = RPW * wid + 8 * j + (lane >> 3);
         okb[j] = (uint32_t)(row * a.ldkv + (((lane & 7) ^ kswz(row)) * 8)) * 2;
         ovb[j] = (uint32_t)(row * a.ldkv + (((lane & 7) ^ vswz(row)) * 8)) * 2;
     }
@@ -135,7 +137,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(4))) vo
         const uint32_t kt = (uint32_t)(k0 * a.ldkv) * 2;  // bytes of the stage's first key row
 #pragma unroll
         for (int j = 0; j < RPW / 8; ++j) {
-            const int r0 = RPW * wave + 8 * j;
+            const int r0 = RPW * wid + 8 * j;
             const uint32_t lk = __builtin_amdgcn_readfirstlane(lk0 + (st * SPB * KT * 64 + r0 * 64) * 2);
             const uint32_t lv = __builtin_amdgcn_readfirstlane(lv0 + (st * SPB * KT * 64 + r0 * 64) * 2);
             asm volatile("buffer_load_dwordx4 %1, %2, 0 offen lds" ::"{m0}"(lk), "v"(okb[j] + kt), "s"(rsk)
@@ -183,6 +185,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(4))) vo
             __syncthreads();
             if (it + SPB < ntk) issue(k0 + SPB * KT, ((it / SPB) + 1) & 1);
         }
+        if (KS > 1 && it % SPB != kgrp) continue;
         const bool skip = !active || (a.window >= 0 && (k0 > qlo + 31 + a.window || k0 + KT - 1 < qlo - a.window));
         if (skip) continue;
         lds_u8* const vt = (lds_u8*)&sV[buf][0];  // this tile's V buffer
@@ -334,6 +337,38 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(4))) vo
         }
     }
 
+    if constexpr (KS > 1) {
+        // Merge in group order.  A group that saw no key of a query has m = -inf,
+        // l = 0 and o = 0, and weighs nothing.
+        float* const part = (float*)smem;  // [group 1 ..][wave][34][lane]
+        __syncthreads();  // every wave is done with the K/V tiles
+        if (kgrp > 0) {
+            float* p = part + ((kgrp - 1) * 4 + wave) * 34 * 64 + lane;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                p[e * 64] = o[0][e];
+                p[(16 + e) * 64] = o[1][e];
+            }
+            p[32 * 64] = m;
+            p[33 * 64] = l;
+        }
+        __syncthreads();
+        if (kgrp > 0) return;
+#pragma unroll
+        for (int g2 = 0; g2 < KS - 1; ++g2) {
+            const float* p = part + (g2 * 4 + wave) * 34 * 64 + lane;
+            const float m2 = p[32 * 64], mn = fmaxf(m, m2);
+            const float w1 = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m - mn) * c);
+            const float w2 = m2 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m2 - mn) * c);
+            l = l * w1 + p[33 * 64] * w2;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                o[0][e] = o[0][e] * w1 + p[e * 64] * w2;
+                o[1][e] = o[1][e] * w1 + p[(16 + e) * 64] * w2;
+            }
+            m = mn;
+        }
+    }
     l += __shfl_xor(l, 32, 64);
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
     if (qi < tile.nq) {
@@ -349,6 +384,55 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(4))) vo
     }
 }
 
+// KS > 1: items whose keys are too few for the split to pay (the launch knows
+// only their number) run as with KS = 1, on the first four waves.  Measured (us,
+// hidden 384, one row of 500 / 900 / 1500 / 3928 keys): KS 1 10.0 / 15.1 / 22.0
+// / 50.4, KS 4 10.9 / 14.3 / 18.6 / 39.0; KS 2 at two items per CU: 8 rows of
+// 900 keys 23.6 -> 23.9, 4 of 1500 31.4 -> 30.3, one of 8192 138 -> 129.
+constexpr int kSplitKeys4 = 832, kSplitKeys2 = 1152;
+
+template <int NW, bool WIN, int KS = 1>
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(4))) void attention_kernel(AttnArgs a) {
+    __shared__ __align__(1024) bf16_t smem[2][NW / 2][KT * 64];
+    // One workgroup per (tile, head), heads varying fastest: callers list the
+    // costliest tiles first, so those are dispatched first, one per CU.
+    const int head = (int)(blockIdx.x % (unsigned)a.heads);
+    const int item = (int)(blockIdx.x / (unsigned)a.heads);
+    AttnTile tile = a.tiles[a.halves ? item >> 1 : item];
+    if (a.halves) {  // this workgroup's 128 queries of a 256-query tile
+        const int off = (item & 1) * 128;
+        if (off >= tile.nq) return;
+        tile.q_row += off;
+        tile.q_pos += off;
+        tile.nq = min(tile.nq - off, 128);
+    }
+    if constexpr (KS > 1) {
+        if (tile.kv_len < (KS == 4 ? kSplitKeys4 : kSplitKeys2)) {
+            if (threadIdx.x >= 256) return;
+            attend<4, WIN, 1>(a, tile, head, *(bf16_t(*)[2][2][KT * 64])smem);
+            return;
+        }
+    }
+    attend<NW, WIN, KS>(a, tile, head, smem);
+}
+
+// Time of `items` 256-query items on `cus` CUs, in units of one at the full rate
+// of a CU that runs two: whole rounds of two per CU, then what is left over.
+// Measured at 8192 / 4096 keys (us, 256-query items against halves): 96 items
+// 69.5 / 51.9 (one 4096-token row, hidden 384), 192 items 136 / 138, 384 items
+// 237 / 221, 576 items 365 / 340, 768 items 400 / 419, 1536 items 774 / 808.
+double wide_cost(long items, long cus) {
+    const long rest = items % (2 * cus);
+    return items / (2 * cus) * 2.0 + (rest == 0 ? 0.0 : rest <= cus ? 1.17 : 2.0);
+}
+
+// The same as 128-query items, four per CU: a CU with one to three of them
+// keeps its SIMDs less busy, but fewer stand idle at the end.
+double halves_cost(long items, long cus) {
+    const long rest = 2 * items % (4 * cus), full = 2 * items / (4 * cus);
+    return full * 2.06 + (rest == 0 ? 0.0 : rest <= cus ? 0.75 : rest <= 2 * cus ? 1.17 : rest <= 3 * cus ? 1.75 : 2.06);
+}
+
 }  // namespace
 
 void launch_attention(const AttnArgs& a, hipStream_t s) {
@@ -359,14 +443,30 @@ void launch_attention(const AttnArgs& a, hipStream_t s) {
     if (a.ldq % 8 || a.ldkv % 8 || a.ldo % 4 || a.ldq < a.heads * 64 || a.ldo < a.heads * 64 ||
         ((uintptr_t)a.q & 15) || ((uintptr_t)a.k & 15) || ((uintptr_t)a.v & 15) || ((uintptr_t)a.out & 7))
         throw jh_error(1, "attention: operands must be 16-byte aligned with row strides % 8 == 0");
-    if ((long)a.ntiles * a.heads > 0x7fffffffL) throw jh_error(1, "attention: grid too large");
-    const dim3 grid((unsigned)(a.ntiles * a.heads));
-    if (a.waves == 8) {
-        if (a.window >= 0) JH_LAUNCH((attention_kernel<8, true>), grid, dim3(512), 0, s, a);
-        else JH_LAUNCH((attention_kernel<8, false>), grid, dim3(512), 0, s, a);
+    if ((long)a.ntiles * a.heads > 0x3fffffffL) throw jh_error(1, "attention: grid too large");
+    AttnArgs b = a;
+    const long cus = gemm_resident_tiles() / 2;
+    long items = (long)a.ntiles * a.heads;
+    bool wide = a.waves == 8;
+    if (wide && (a.window >= 0 || halves_cost(items, cus) < wide_cost(items, cus))) {
+        b.halves = 1;
+        wide = false;
+        items *= 2;
+    }
+    // Few items leave SIMDs with one or two waves, or none: full attention over
+    // long rows then splits each item's keys over two or four times the waves.
+    // (Not window layers: an item has at most four or five key tiles.)
+    const int ks = wide || !a.key_split || a.window >= 0 ? 1 : items <= cus ? 4 : items <= 2 * cus ? 2 : 1;
+    const dim3 grid((unsigned)items);
+    if (wide) {
+        JH_LAUNCH((attention_kernel<8, false>), grid, dim3(512), 0, s, b);
+    } else if (ks == 4) {
+        JH_LAUNCH((attention_kernel<16, false, 4>), grid, dim3(1024), 0, s, b);
+    } else if (ks == 2) {
+        JH_LAUNCH((attention_kernel<8, false, 2>), grid, dim3(512), 0, s, b);
     } else {
-        if (a.window >= 0) JH_LAUNCH((attention_kernel<4, true>), grid, dim3(256), 0, s, a);
-        else JH_LAUNCH((attention_kernel<4, false>), grid, dim3(256), 0, s, a);
+        if (a.window >= 0) JH_LAUNCH((attention_kernel<4, true>), grid, dim3(256), 0, s, b);
+        else JH_LAUNCH((attention_kernel<4, false>), grid, dim3(256), 0, s, b);
     }
     HIP_CHECK(hipGetLastError());
 }

@@ -524,6 +524,7 @@ struct jh_model {
                    long ldo, const AttnTile* tiles, size_t n, int nheads, int window, double pairs, double qrows,
                    int waves = 4) {
         AttnArgs a{q, ldq, k, v, ldkv, out, ldo, tiles, (int)n, nheads, window, 0.125f * 1.4426950408889634f, waves};
+        a.key_split = use_splitk;
         const double hd = 64.0 * nheads;
         timed(cls, 4.0 * hd * pairs, qrows * hd * 2 * 2 + (double)T * hd * 2 * 2, [&] { launch_attention(a, stream); });
         if (profiling && !replay[cls]) replay[cls] = [a, st = stream] { launch_attention(a, st); };

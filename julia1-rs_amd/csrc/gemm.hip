@@ -1351,6 +1351,8 @@ bool validate_gemm(int epi, const GemmArgs& a) {
 
 }  // namespace
 
+int gemm_resident_tiles() { return resident_tiles(); }
+
 bool validate_gemm_args(int epi, const GemmArgs& a) { return validate_gemm(epi, a); }
 
 int gemm_splitk_count(int epi, const GemmArgs& a) {

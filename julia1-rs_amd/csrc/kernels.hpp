@@ -86,6 +86,10 @@ int gemm_ws_block_tokens();
 void launch_gemm_ws(int epilogue, const GemmArgs& a, hipStream_t stream);
 void pack_ws(const bf16_t* w, int n, int k, bf16_t* out);
 
+// 256-thread workgroups with at most 80 KB of LDS that the current device
+// holds at once (two per CU), a multiple of its 8 XCDs.
+int gemm_resident_tiles();
+
 struct AttnTile {
     int32_t q_row, nq, kv_row, kv_len, q_pos;
 };
@@ -104,6 +108,8 @@ struct AttnArgs {
     int window;        // < 0: global
     float scale_log2;  // softmax scale · log2(e)
     int waves = 4;     // waves per work item: 4 (tiles of <= 128 queries) or 8 (<= 256 queries)
+    bool key_split = true;  // few items may share the keys of a query among several waves
+    int halves = 0;    // set by launch_attention: two 128-query workgroups per 256-query tile
 };
 
 void launch_attention(const AttnArgs& a, hipStream_t stream);

@@ -714,6 +714,39 @@ def test_attention_full_length_8192(window):
     assert worst < 2e-2, worst
 
 
+@pytest.mark.parametrize("rate", [0.0, 0.4])
+@pytest.mark.parametrize("heads,lens,wide", [
+    (2, [831, 832, 833, 960, 1], False),   # at most one item per CU: keys split four ways from 832 on
+    (12, [1151, 1152, 1153, 130], False),  # up to two per CU: two ways from 1152 on
+    (12, [1407, 1300], True),              # 256-query tiles run as two 128-query workgroups each
+])
+def test_attention_key_split(heads, lens, wide, rate):
+    """Few work items over long rows: groups of waves take every second or fourth key tile and merge their running
+    maxima, sums and outputs.  With `rate`, scores climb along the row (log2 units per key tile), so the groups'
+    maxima differ and a group may hold almost all of the weight.  Each output is a weighted mean of v with P and
+    the result rounded to bf16 (2^-9 each) and scores summed in FP32, so its error is within 2^-8 max|v|."""
+    r = rng(57)
+    h = heads * 64
+    t = sum(lens)
+    q = np.abs(r.standard_normal((t, h))) + 0.5
+    u = np.abs(r.standard_normal(h)) + 0.5
+    k = 0.3 * r.standard_normal((t, h))
+    v = r.standard_normal((t, h))
+    seqs, start = [], 0
+    for ln in lens:
+        k[start:start + ln] += (rate * np.arange(ln) / 64.0)[:, None] * u[None, :] / 16
+        seqs.append((start, ln, start, ln, 0))
+        start += ln
+    qkv = bf16_round(np.concatenate([q, k, v], 1).astype(np.float32))
+    expect = _attn_ref64(qkv[:, :h], qkv[:, h:2 * h], qkv[:, 2 * h:], seqs, heads, -1)
+    dq = dev(qkv, BF16)
+    out = torch.zeros(t, h, dtype=BF16, device="cuda")
+    hip.op_attention(dq, 3 * h, dq[:, h:], dq[:, 2 * h:], 3 * h, out, h,
+                     dev(np.array(_tiles(lens, 256 if wide else 128), dtype=np.int32)), heads, -1, wide=wide)
+    assert np.abs(qkv[:, 2 * h:]).max() < 5.5
+    assert np.abs(host(out) - expect).max() < 2.0 ** -8 * 5.5, np.abs(host(out) - expect).max()
+
+
 def test_attention_marker_queries():
     """Queries from a separate buffer (the marker-only head layer) against full keys."""
     r = rng(10)
