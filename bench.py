@@ -109,10 +109,10 @@ def committed_traffic(kernel, workload):
 
 
 # Kernel classes whose launches have a kernel symbol of their own in a config1 forward, so their counters can
-# be told apart in a rocprofv3 run (the Wo class shares gemm_ws_kernel<3> with the head's out_proj, and the
+# be told apart in a rocprofv3 run (the Wo class shares gemm_ws_kernel<3, false> with the head's out_proj, and the
 # attention classes share attention_kernel).
-TRAFFIC_SYMBOL = {"gemm_qkv_rope": "gemm_ws_kernel<1>", "gemm_wi_geglu": "gemm_ws_kernel<2>",
-                  "gemm_wo2_resid": "gemm_ws2_kernel<36>"}
+TRAFFIC_SYMBOL = {"gemm_qkv_rope": "gemm_ws_kernel<1", "gemm_wi_geglu": "gemm_ws_kernel<2",
+                  "gemm_wo2_resid": "gemm_ws2_kernel<36"}
 
 
 def counter_bytes(rows, copy_mib=256, replays=51):

@@ -58,8 +58,10 @@ int jh_op_gemm(int epilogue, const void* x, size_t ldx, const int32_t* gather, s
  * tile count, as the backend does for small batches) whose FP32 partial sums
  * go to `workspace` (splits · rows · N floats must fit `workspace_bytes`;
  * fewer splits are used otherwise), then one more kernel sums them in chunk
- * order and applies the epilogue.  Deterministic.  Same requirements as
- * jh_op_gemm.  No reference counterpart (cuBLAS chooses its own split-K).
+ * order and applies the epilogue.  With splits 0, shapes that a one-launch
+ * kernel serves better (few tokens; K = 384, 768 or 1152 from some hundreds of
+ * tokens up) run on it without the workspace.  Deterministic.  Same
+ * requirements as jh_op_gemm.  No reference counterpart (cuBLAS chooses its own split-K).
  */
 int jh_op_gemm_splitk(int epilogue, const void* x, size_t ldx, const int32_t* gather, size_t rows,
                       const void* w, size_t n, size_t k, void* out, size_t ldo, size_t col,

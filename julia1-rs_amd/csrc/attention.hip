@@ -384,22 +384,23 @@ __device__ __forceinline__ void attend(const AttnArgs& a, const AttnTile& tile, 
     }
 }
 
-// KS > 1: items whose keys are too few for the split to pay (the launch knows
-// only their number) run as with KS = 1, on the first four waves.  Measured (us,
+// KS > 1: items whose keys are too few for the split to pay (a caller that knows
+// of none as long says so in key_split) run as with KS = 1, on the first four waves.  Measured (us,
 // hidden 384, one row of 500 / 900 / 1500 / 3928 keys): KS 1 10.0 / 15.1 / 22.0
 // / 50.4, KS 4 10.9 / 14.3 / 18.6 / 39.0; KS 2 at two items per CU: 8 rows of
 // 900 keys 23.6 -> 23.9, 4 of 1500 31.4 -> 30.3, one of 8192 138 -> 129.
-constexpr int kSplitKeys4 = 832, kSplitKeys2 = 1152;
+constexpr int kSplitKeys4 = ATTN_SPLIT_KEYS, kSplitKeys2 = 1152;
 
-template <int NW, bool WIN, int KS = 1>
+// HALVES: two workgroups per 256-query tile, each with 128 of its queries.
+template <int NW, bool WIN, int KS = 1, bool HALVES = false>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(4))) void attention_kernel(AttnArgs a) {
     __shared__ __align__(1024) bf16_t smem[2][NW / 2][KT * 64];
     // One workgroup per (tile, head), heads varying fastest: callers list the
     // costliest tiles first, so those are dispatched first, one per CU.
     const int head = (int)(blockIdx.x % (unsigned)a.heads);
     const int item = (int)(blockIdx.x / (unsigned)a.heads);
-    AttnTile tile = a.tiles[a.halves ? item >> 1 : item];
-    if (a.halves) {  // this workgroup's 128 queries of a 256-query tile
+    AttnTile tile = a.tiles[HALVES ? item >> 1 : item];
+    if constexpr (HALVES) {
         const int off = (item & 1) * 128;
         if (off >= tile.nq) return;
         tile.q_row += off;
@@ -433,6 +434,14 @@ double halves_cost(long items, long cus) {
     return full * 2.06 + (rest == 0 ? 0.0 : rest <= cus ? 0.75 : rest <= 2 * cus ? 1.17 : rest <= 3 * cus ? 1.75 : 2.06);
 }
 
+template <bool HALVES>
+void launch_items(const AttnArgs& a, int ks, dim3 grid, hipStream_t s) {
+    if (ks == 4) JH_LAUNCH((attention_kernel<16, false, 4, HALVES>), grid, dim3(1024), 0, s, a);
+    else if (ks == 2) JH_LAUNCH((attention_kernel<8, false, 2, HALVES>), grid, dim3(512), 0, s, a);
+    else if (a.window >= 0) JH_LAUNCH((attention_kernel<4, true, 1, HALVES>), grid, dim3(256), 0, s, a);
+    else JH_LAUNCH((attention_kernel<4, false, 1, HALVES>), grid, dim3(256), 0, s, a);
+}
+
 }  // namespace
 
 void launch_attention(const AttnArgs& a, hipStream_t s) {
@@ -444,12 +453,11 @@ void launch_attention(const AttnArgs& a, hipStream_t s) {
         ((uintptr_t)a.q & 15) || ((uintptr_t)a.k & 15) || ((uintptr_t)a.v & 15) || ((uintptr_t)a.out & 7))
         throw jh_error(1, "attention: operands must be 16-byte aligned with row strides % 8 == 0");
     if ((long)a.ntiles * a.heads > 0x3fffffffL) throw jh_error(1, "attention: grid too large");
-    AttnArgs b = a;
     const long cus = gemm_resident_tiles() / 2;
     long items = (long)a.ntiles * a.heads;
-    bool wide = a.waves == 8;
+    bool wide = a.waves == 8, halves = false;
     if (wide && (a.window >= 0 || halves_cost(items, cus) < wide_cost(items, cus))) {
-        b.halves = 1;
+        halves = true;
         wide = false;
         items *= 2;
     }
@@ -458,15 +466,8 @@ void launch_attention(const AttnArgs& a, hipStream_t s) {
     // (Not window layers: an item has at most four or five key tiles.)
     const int ks = wide || !a.key_split || a.window >= 0 ? 1 : items <= cus ? 4 : items <= 2 * cus ? 2 : 1;
     const dim3 grid((unsigned)items);
-    if (wide) {
-        JH_LAUNCH((attention_kernel<8, false>), grid, dim3(512), 0, s, b);
-    } else if (ks == 4) {
-        JH_LAUNCH((attention_kernel<16, false, 4>), grid, dim3(1024), 0, s, b);
-    } else if (ks == 2) {
-        JH_LAUNCH((attention_kernel<8, false, 2>), grid, dim3(512), 0, s, b);
-    } else {
-        if (a.window >= 0) JH_LAUNCH((attention_kernel<4, true>), grid, dim3(256), 0, s, b);
-        else JH_LAUNCH((attention_kernel<4, false>), grid, dim3(256), 0, s, b);
-    }
+    if (wide) JH_LAUNCH((attention_kernel<8, false>), grid, dim3(512), 0, s, a);
+    else if (halves) launch_items<true>(a, ks, grid, s);
+    else launch_items<false>(a, ks, grid, s);
     HIP_CHECK(hipGetLastError());
 }

@@ -202,6 +202,7 @@ struct jh_model {
     // staged batch
     bool staged = false;
     size_t T = 0, S = 0, M = 0, ntiles = 0, nmtiles = 0;
+    uint32_t longest = 0;  // tokens of the longest sequence
     uint32_t* d_ids = nullptr;
     uint32_t* d_tok = nullptr;
     AttnTile* d_tiles = nullptr;
@@ -436,6 +437,7 @@ struct jh_model {
         M = m;
         ntiles = tiles.size();
         nmtiles = mtiles.size();
+        longest = nseq ? *std::max_element(lens, lens + nseq) : 0;
         staged = true;
     }
 
@@ -464,6 +466,7 @@ struct jh_model {
         GemmArgs a{(const bf16_t*)xp, ldx, nullptr, (int)rows, w, H, k, xo, H, 0, bias,
                    (const int32_t*)d_tok, nullptr, nullptr, 0};
         int S = 1;
+        a.w_ws = w_ws;
         if (use_splitk) {
             a.partial = splitk.as<float>();
             a.partial_bytes = kSplitkBytes;
@@ -524,7 +527,7 @@ struct jh_model {
                    long ldo, const AttnTile* tiles, size_t n, int nheads, int window, double pairs, double qrows,
                    int waves = 4) {
         AttnArgs a{q, ldq, k, v, ldkv, out, ldo, tiles, (int)n, nheads, window, 0.125f * 1.4426950408889634f, waves};
-        a.key_split = use_splitk;
+        a.key_split = use_splitk && longest >= (uint32_t)ATTN_SPLIT_KEYS;
         const double hd = 64.0 * nheads;
         timed(cls, 4.0 * hd * pairs, qrows * hd * 2 * 2 + (double)T * hd * 2 * 2, [&] { launch_attention(a, stream); });
         if (profiling && !replay[cls]) replay[cls] = [a, st = stream] { launch_attention(a, st); };
@@ -676,7 +679,8 @@ struct jh_model {
             return;
         }
         MetaSlot& ms = slots[cur];
-        const size_t key[8] = {T, M, S, ntiles, nmtiles, (size_t)ws_gen, nglong, ngshort};
+        const size_t key[8] = {T, M, S, ntiles, nmtiles, (size_t)ws_gen, nglong,
+                               2 * ngshort + (longest >= (uint32_t)ATTN_SPLIT_KEYS)};
         if (!ms.graph || !std::equal(key, key + 8, ms.graph_key)) {
             // Capturing and instantiating the ~200-launch forward costs ~0.5 ms
             // on MI355X while replay saves nothing measurable over eager

@@ -1168,6 +1168,57 @@ int small_bf(int epi, const GemmArgs& a) {
     return a.k <= small_kmax<64>() ? 64 : 0;
 }
 
+// Waves per workgroup of the slab-resident kernel (K = 384) for `a`, or 0 when
+// launch_gemm does not use it.  It sums K in steps of 32, the tiled kernels in
+// steps of 16, so like the small-batch paths it is left out when a row must not
+// depend on the batch (no workspace).  Measured (us, tiled or small-batch kernel
+// against this one), by N and tokens:
+//   N = 384: 933 4.2 / 5.3, 1500 7.1 / 6.7, 3300 10.6 / 7.4, 4323 13.2 / 7.9,
+//     7556 10.6 / 10.2, 16384 14.5 / 13.7, 65536 58.8 / 55.6: from the second
+//     round of the small-batch kernel's 64 x 32 tiles on (one per CU);
+//   N = 1152: 600 6.7 / 7.3, 933 8.8 / 7.6, 1500 12.0 / 7.8, 2500 9.5 / 9.8,
+//     4323 12.2 / 12.7; N = 2304: 400 6.4 / 7.7, 600 8.7 / 7.9, 1500 8.3 / 9.6:
+//     from the small-batch kernel's third round to its last;
+//   twelve waves (384-row slabs), N = 1152: 9500 15.5 / 17.7, 16384 24.0 / 24.0,
+//     65536 96 / 66; N = 2304: 16384 38.9 / 37.1, 65536 167 / 124.
+int slab_waves(const GemmArgs& a) {
+    if (!a.partial || a.splits != 0 || !gemm_slab_supported(a)) return 0;
+    if (a.rows >= 16384 && a.n >= 1024 && a.n % 384 == 0) return 12;
+    const long cus = resident_tiles() / 2, tiles = (long)((a.n + 127) / 128) * ((a.rows + 127) / 128);
+    const long small = (long)(a.n / 64) * ((a.rows + SMALL_BT - 1) / SMALL_BT);
+    if (a.n < 1024) return small > cus ? 4 : 0;
+    return tiles < 128 && small > 2 * cus ? 4 : 0;
+}
+
+// Whether launch_gemm runs `a` on the weight-stationary kernel (K = 768, or 1152
+// with the residual epilogue).  Without a workspace: whenever W comes packed for
+// it, for every token count, so that a row's sums run in one order whatever else
+// is in the batch (the tiled kernels step K by 16, this one by 32, so switching
+// kernels on the batch size would move a row's outputs by FP32 rounding).  With
+// one: as soon as the small-batch kernel's tiles (one per CU) need a second round.
+// Measured (us, small-batch or split-K kernels against this one, packed):
+//   K = 768, N = 768 (64-feature tiles: 672 tokens a round): 500 5.8 / 7.6,
+//     700 9.3 / 7.9, 1500 13.3 / 8.7, 2500 17.0 / 10.4;
+//   K = 768, N = 2304 (224 tokens): 300 8.8 / 8.0, 500 12.4 / 9.6, 700 15.8 / 10.1;
+//     N = 3072 (160 tokens): 180 9.3 / 9.8, so a little later for wide outputs;
+//   K = 1152 (32-feature tiles), N = 768 (320 tokens): 300 4.8 / 7.0, 500 16.5 /
+//     7.1, 2500 22.3 / 12.2; N = 384 (672 tokens): 500 5.1 / 6.0, 700 13.8 / 6.1,
+//     4323 22.3 / 11.2.
+// W as it lies, row-major, takes 0.5 to 1.5 us longer to fetch, which moves the
+// lines: N = 2304, small-batch or tiled kernel against this one: 300 8.8 / 9.4,
+// 500 12.4 / 11.1, 2500 17.2 / 17.0, 3300 18.6 / 19.8, 4323 21.6 / 22.2, 6000
+// 30.8 / 27.5; K = 1152, N = 768: 7556 22.4 / 19.8, 16384 45.6 / 47.2.
+bool ws_takes(int epi, const GemmArgs& a) {
+    if (!a.partial) return gemm_ws_supported(epi, a);
+    if (!gemm_ws_shape(epi, a) || (a.w_ws && !gemm_ws_supported(epi, a))) return false;
+    const long cus = resident_tiles() / 2, tiles = (long)((a.n + 127) / 128) * ((a.rows + 127) / 128);
+    const long small = (long)(a.n / (a.k <= small_kmax<64>() ? 64 : 32)) * ((a.rows + SMALL_BT - 1) / SMALL_BT);
+    if (a.w_ws) return a.n < 1024 || a.k > small_kmax<64>() ? small > cus : 4 * small > 5 * cus;
+    if (a.k > small_kmax<64>()) return small > cus && (long)a.rows * a.n < 12288L * 768;
+    if (a.n < 1024) return small > cus;
+    return tiles < 128 ? 2 * small > 3 * cus : a.rows >= 6000;
+}
+
 template <int EPI>
 void launch_small(const GemmArgs& a, int bf, hipStream_t s) {
     constexpr bool PAIRED = EPI == JH_EPI_ROPE_BF16 || EPI == JH_EPI_GEGLU_BF16;
@@ -1270,6 +1321,14 @@ template <int EPI>
 void launch_cfg(const GemmArgs& a, hipStream_t s) {
     constexpr int BF = 128, BT = 128;
     const int blocks = ((a.n + BF - 1) / BF) * ((a.rows + BT - 1) / BT);
+    if (const int waves = slab_waves(a)) {
+        launch_gemm_slab(EPI, a, waves, s);
+        return;
+    }
+    if (a.splits == 0 && ws_takes(EPI, a)) {
+        launch_gemm_ws(EPI, a, s);
+        return;
+    }
     if (const int bf = small_bf(EPI, a)) {
         launch_small<EPI>(a, bf, s);
         return;
@@ -1287,11 +1346,7 @@ void launch_cfg(const GemmArgs& a, hipStream_t s) {
         HIP_CHECK(hipGetLastError());
         return;
     }
-    // Weight-stationary kernel whenever W comes packed for it, for every
-    // token count: a row's sums then run in one order whatever else is in the
-    // batch (the tiled kernels step K by 16, this one by 32, so switching
-    // kernels on the batch size would move a row's outputs by FP32 rounding).
-    if (gemm_ws_supported(EPI, a)) {
+    if (gemm_ws_supported(EPI, a)) {  // a forced split count that K does not allow
         launch_gemm_ws(EPI, a, s);
         return;
     }
@@ -1356,7 +1411,7 @@ int gemm_resident_tiles() { return resident_tiles(); }
 bool validate_gemm_args(int epi, const GemmArgs& a) { return validate_gemm(epi, a); }
 
 int gemm_splitk_count(int epi, const GemmArgs& a) {
-    if (!validate_gemm(epi, a)) return 1;
+    if (!validate_gemm(epi, a) || slab_waves(a) || (a.splits == 0 && ws_takes(epi, a))) return 1;
     return splitk_count(a, (long)((a.n + 127) / 128) * ((a.rows + 127) / 128));
 }
 

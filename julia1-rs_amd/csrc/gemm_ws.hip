@@ -70,7 +70,46 @@ __device__ constexpr int swz(int r) { return (r >> 1) & 7; }
 // read (tokens 4kg + i of four kg, sixteen columns each) cover all banks.
 __device__ inline int old_token(int lane) { return 4 * ((lane >> 2) & 3) + (lane >> 4); }
 
-template <int EPI>
+// A wave's W fragments from row-major W: NSEG 128-byte segments of two groups of
+// 16 rows (HSTEP rows apart), read eight whole segments per load so that adjacent
+// lanes read adjacent memory (in the fragments' own lane order, 16 rows side by
+// side, the loads ran at 36 instead of 120 B/ns per CU), and turned into
+// fragments through 2 KB of LDS of the wave's own (a wave's LDS operations
+// complete in order, so it is reused without a wait).  `wp`: this lane's part of
+// the first load.  Four segments are in flight; put(s, h, fragment) takes slice
+// s of group h.
+template <int NSEG, int HSTEP, class Put>
+__device__ __forceinline__ void row_fragments(const bf16_t* wp, int k, bf16_t* sw, int lane, Put put) {
+    constexpr int AHEAD = 4;
+    u32x4 wr[AHEAD][4];
+    auto load = [&](int j) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            wr[j % AHEAD][i] = *(const u32x4*)(wp + (long)((i >> 1) * HSTEP + (i & 1) * 8) * k + j * 64);
+    };
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) load(j);
+#pragma unroll
+    for (int j = 0; j < NSEG; ++j) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int row = 8 * i + (lane >> 3);
+                *(u32x4*)&sw[row * 64 + (((lane & 7) ^ swz(row)) * 8)] = wr[j % AHEAD][2 * h + i];
+            }
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+                put(2 * j + e, h,
+                    *(const bf16x8*)&sw[(lane & 15) * 64 + (((4 * e + (lane >> 4)) ^ swz(lane & 15)) * 8)]);
+        }
+        if (j + AHEAD < NSEG) load(j + AHEAD);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// ROWS: W is row-major (a.w) instead of packed (a.w_ws).
+template <int EPI, bool ROWS>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void gemm_ws_kernel(GemmArgs a, int nF,
                                                                                                int R, int nTB) {
     constexpr bool ROPE = EPI == JH_EPI_ROPE_BF16;
@@ -193,26 +232,38 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
     }
     __syncthreads();
     bf16x8 wf[WS_SR][2];
-    const bf16_t* wp = a.w_ws + (long)(f * 8 + wave) * WS_S * 2 * 512;
+    if constexpr (ROWS) {
+        // through the second X slot, which the first block refills
+        bf16_t* const own = swl + wave * WS_SL * 2 * 512 + lane * 8;
+        row_fragments<WS_S / 2, 32>(a.w + (long)(64 * (4 * f + (wave >> 1)) + 16 * (wave & 1) + (lane >> 3)) * WS_K +
+                                        (lane & 7) * 8,
+                                    WS_K, sx + WS_XSLOT + wave * 1024, lane, [&](int sl, int h, bf16x8 v) {
+                                        if (sl < WS_SR) wf[sl < WS_SR ? sl : 0][h] = v;
+                                        else *(bf16x8*)&own[((sl - WS_SR) * 2 + h) * 512] = v;
+                                    });
+    } else {
+        const bf16_t* wp = a.w_ws + (long)(f * 8 + wave) * WS_S * 2 * 512;
 #pragma unroll
-    for (int s = 0; s < WS_SR; ++s)
+        for (int s = 0; s < WS_SR; ++s)
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            wf[s][h] = *(const bf16x8*)(wp + (s * 2 + h) * 512 + lane * 8);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    if constexpr (WS_SL > 0) {
-        const i32x4 rw = make_rsrc(wp + WS_SR * 2 * 512, WS_SL * 2 * 1024);
+            for (int h = 0; h < 2; ++h) {
+                wf[s][h] = *(const bf16x8*)(wp + (s * 2 + h) * 512 + lane * 8);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        if constexpr (WS_SL > 0) {
+            const i32x4 rw = make_rsrc(wp + WS_SR * 2 * 512, WS_SL * 2 * 1024);
 #pragma unroll
-        for (int j = 0; j < WS_SL * 2; ++j) {
-            const uint32_t m0 =
-                __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)&swl[(wave * WS_SL * 2 + j) * 512]);
-            asm volatile("buffer_load_dwordx4 %1, %2, %3 offen lds" ::"{m0}"(m0), "v"((uint32_t)lane * 16), "s"(rw),
-                         "s"(j * 1024)
-                         : "memory");
+            for (int j = 0; j < WS_SL * 2; ++j) {
+                const uint32_t m0 =
+                    __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)&swl[(wave * WS_SL * 2 + j) * 512]);
+                asm volatile("buffer_load_dwordx4 %1, %2, %3 offen lds" ::"{m0}"(m0), "v"((uint32_t)lane * 16), "s"(rw),
+                             "s"(j * 1024)
+                             : "memory");
+            }
         }
     }
-    // the first block's X, positions and bias landed (48 W loads and DMAs since)
+    // the first block's X, positions and bias landed (packed W: 48 W loads and DMAs since;
+    // row-major W: every load was waited for)
     asm volatile("s_waitcnt vmcnt(48)" ::: "memory");
     __syncthreads();
 
@@ -482,7 +533,7 @@ constexpr int W2_K = 1152;
 constexpr int W2_ROWS = 128;             // W rows per workgroup
 constexpr int W2_PD = 6;                 // B-fragment reads in flight
 
-template <int KS>  // 32-deep K slices
+template <int KS, bool ROWS>  // 32-deep K slices; W row-major (a.w) instead of packed (a.w_ws)
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void gemm_ws2_kernel(GemmArgs a, int nF,
                                                                                                 int R, int nTB) {
     constexpr int W2_K = KS * 32;
@@ -546,14 +597,22 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
     }
     __syncthreads();
     bf16x8 wf[W2_SH][2];
-    const bf16_t* wp = a.w_ws + (long)(f * 8 + wave) * W2_SH * 2 * 512;
+    if constexpr (ROWS) {
+        // through the second X slot, which the first block refills
+        row_fragments<W2_SH / 2, 16>(a.w + (long)(W2_ROWS * f + 32 * rg + (lane >> 3)) * W2_K + 32 * W2_SH * kh +
+                                         (lane & 7) * 8,
+                                     W2_K, sx + W2_XSLOT + wave * 1024, lane,
+                                     [&](int sl, int h, bf16x8 v) { wf[sl][h] = v; });
+    } else {
+        const bf16_t* wp = a.w_ws + (long)(f * 8 + wave) * W2_SH * 2 * 512;
 #pragma unroll
-    for (int s = 0; s < W2_SH; ++s)
+        for (int s = 0; s < W2_SH; ++s)
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            wf[s][h] = *(const bf16x8*)(wp + (s * 2 + h) * 512 + lane * 8);
-            __builtin_amdgcn_sched_barrier(0);
-        }
+            for (int h = 0; h < 2; ++h) {
+                wf[s][h] = *(const bf16x8*)(wp + (s * 2 + h) * 512 + lane * 8);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+    }
     // the first block's X and the bias landed (the 36 W loads issued since may not have)
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * W2_SH) : "memory");
     __syncthreads();
@@ -710,10 +769,14 @@ int device_cus() {
 
 }  // namespace
 
-bool gemm_ws_supported(int epi, const GemmArgs& a) {
-    if (!a.w_ws || a.gather || a.xf || a.rows <= 0 || ((uintptr_t)a.w_ws & 15)) return false;
+bool gemm_ws_shape(int epi, const GemmArgs& a) {
+    if (a.gather || a.xf || a.rows <= 0) return false;
     if (a.k == W2_K) return a.n % W2_ROWS == 0 && epi == JH_EPI_RESID_F32;
     return a.k == WS_K && a.n % WS_ROWS == 0 && epi >= JH_EPI_STORE_BF16 && epi <= JH_EPI_BIAS_F32;
+}
+
+bool gemm_ws_supported(int epi, const GemmArgs& a) {
+    return a.w_ws && !((uintptr_t)a.w_ws & 15) && gemm_ws_shape(epi, a);
 }
 
 // W rows per workgroup of the kernel that takes K.
@@ -727,30 +790,36 @@ int gemm_ws_ranges(const GemmArgs& a) {
 
 int gemm_ws_block_tokens() { return WS_TB; }
 
-void launch_gemm_ws(int epi, const GemmArgs& a, hipStream_t s) {
-    if (!gemm_ws_supported(epi, a))
-        throw jh_error(1, "gemm: weight-stationary kernel needs packed W and K = 768 with N % 256 == 0, or K = 1152 "
-                          "with N % 128 == 0 and the residual epilogue");
+template <bool ROWS>
+static void launch_ws(int epi, const GemmArgs& a, hipStream_t s) {
     const int nF = a.n / ws_rows(a.k), nTB = (a.rows + WS_TB - 1) / WS_TB, R = gemm_ws_ranges(a);
     const dim3 grid((unsigned)(nF * R)), block(512);
     if (a.k == W2_K) {
-        JH_LAUNCH((gemm_ws2_kernel<W2_K / 32>), grid, block, 0, s, a, nF, R, nTB);
+        JH_LAUNCH((gemm_ws2_kernel<W2_K / 32, ROWS>), grid, block, 0, s, a, nF, R, nTB);
         HIP_CHECK(hipGetLastError());
         return;
     }
     switch (epi) {
-        case JH_EPI_STORE_BF16: JH_LAUNCH((gemm_ws_kernel<JH_EPI_STORE_BF16>), grid, block, 0, s, a, nF, R, nTB); break;
-        case JH_EPI_ROPE_BF16: JH_LAUNCH((gemm_ws_kernel<JH_EPI_ROPE_BF16>), grid, block, 0, s, a, nF, R, nTB); break;
-        case JH_EPI_GEGLU_BF16: JH_LAUNCH((gemm_ws_kernel<JH_EPI_GEGLU_BF16>), grid, block, 0, s, a, nF, R, nTB); break;
-        case JH_EPI_RESID_F32: JH_LAUNCH((gemm_ws_kernel<JH_EPI_RESID_F32>), grid, block, 0, s, a, nF, R, nTB); break;
-        case JH_EPI_BIAS_BF16: JH_LAUNCH((gemm_ws_kernel<JH_EPI_BIAS_BF16>), grid, block, 0, s, a, nF, R, nTB); break;
+        case JH_EPI_STORE_BF16: JH_LAUNCH((gemm_ws_kernel<JH_EPI_STORE_BF16, ROWS>), grid, block, 0, s, a, nF, R, nTB); break;
+        case JH_EPI_ROPE_BF16: JH_LAUNCH((gemm_ws_kernel<JH_EPI_ROPE_BF16, ROWS>), grid, block, 0, s, a, nF, R, nTB); break;
+        case JH_EPI_GEGLU_BF16: JH_LAUNCH((gemm_ws_kernel<JH_EPI_GEGLU_BF16, ROWS>), grid, block, 0, s, a, nF, R, nTB); break;
+        case JH_EPI_RESID_F32: JH_LAUNCH((gemm_ws_kernel<JH_EPI_RESID_F32, ROWS>), grid, block, 0, s, a, nF, R, nTB); break;
+        case JH_EPI_BIAS_BF16: JH_LAUNCH((gemm_ws_kernel<JH_EPI_BIAS_BF16, ROWS>), grid, block, 0, s, a, nF, R, nTB); break;
         case JH_EPI_BIAS_RELU_BF16:
-            JH_LAUNCH((gemm_ws_kernel<JH_EPI_BIAS_RELU_BF16>), grid, block, 0, s, a, nF, R, nTB);
+            JH_LAUNCH((gemm_ws_kernel<JH_EPI_BIAS_RELU_BF16, ROWS>), grid, block, 0, s, a, nF, R, nTB);
             break;
-        case JH_EPI_BIAS_F32: JH_LAUNCH((gemm_ws_kernel<JH_EPI_BIAS_F32>), grid, block, 0, s, a, nF, R, nTB); break;
+        case JH_EPI_BIAS_F32: JH_LAUNCH((gemm_ws_kernel<JH_EPI_BIAS_F32, ROWS>), grid, block, 0, s, a, nF, R, nTB); break;
         default: throw jh_error(1, "gemm: unknown epilogue");
     }
     HIP_CHECK(hipGetLastError());
+}
+
+void launch_gemm_ws(int epi, const GemmArgs& a, hipStream_t s) {
+    if (!(a.w_ws ? gemm_ws_supported(epi, a) : gemm_ws_shape(epi, a) && a.w))
+        throw jh_error(1, "gemm: weight-stationary kernel needs packed W and K = 768 with N % 256 == 0, or K = 1152 "
+                          "with N % 128 == 0 and the residual epilogue");
+    if (a.w_ws) launch_ws<false>(epi, a, s);
+    else launch_ws<true>(epi, a, s);
 }
 
 // Host-side packing of a bf16 [n, k] row-major W into the weight-stationary

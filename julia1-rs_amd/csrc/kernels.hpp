@@ -78,6 +78,8 @@ void launch_gemm_partial(int epilogue, const GemmArgs& a, int splits, hipStream_
 // no gather or LayerNorm prologue.  gemm_ws_ranges is the number of token
 // ranges each 256-row slab is split into (one workgroup per CU).
 bool gemm_ws_supported(int epilogue, const GemmArgs& a);
+// The same but for W: launch_gemm_ws reads a.w, row-major, where a.w_ws is null.
+bool gemm_ws_shape(int epilogue, const GemmArgs& a);
 // The shape, alignment and argument checks of launch_gemm (throws jh_error);
 // false when there is nothing to do (rows == 0).
 bool validate_gemm_args(int epilogue, const GemmArgs& a);
@@ -86,6 +88,10 @@ int gemm_ws_block_tokens();
 void launch_gemm_ws(int epilogue, const GemmArgs& a, hipStream_t stream);
 void pack_ws(const bf16_t* w, int n, int k, bf16_t* out);
 
+// Slab-resident kernel (gemm_slab.hip): K = 384, N % 128 == 0, no gather or
+// LayerNorm prologue; every epilogue.  `waves` per workgroup: 4, or 12 (N % 384 == 0).
+bool gemm_slab_supported(const GemmArgs& a);
+void launch_gemm_slab(int epi, const GemmArgs& a, int waves, hipStream_t stream);
 // 256-thread workgroups with at most 80 KB of LDS that the current device
 // holds at once (two per CU), a multiple of its 8 XCDs.
 int gemm_resident_tiles();
@@ -108,9 +114,9 @@ struct AttnArgs {
     int window;        // < 0: global
     float scale_log2;  // softmax scale · log2(e)
     int waves = 4;     // waves per work item: 4 (tiles of <= 128 queries) or 8 (<= 256 queries)
-    bool key_split = true;  // few items may share the keys of a query among several waves
-    int halves = 0;    // set by launch_attention: two 128-query workgroups per 256-query tile
+    bool key_split = true;  // few items with ATTN_SPLIT_KEYS keys or more may share a query's keys among several waves
 };
+constexpr int ATTN_SPLIT_KEYS = 832;
 
 void launch_attention(const AttnArgs& a, hipStream_t stream);
 
