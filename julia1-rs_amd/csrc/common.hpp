@@ -63,25 +63,48 @@ __device__ inline i32x4 make_rsrc(const void* base, uint64_t bytes) {
                  (int)(uint32_t)(bytes < 0xffffffffull ? bytes : 0xffffffffull), 0x00020000};
 }
 
-__device__ inline float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, JH_WAVE);
-    return v;
+// v plus the same value of another lane, lanes paired as in a butterfly over 1, 2,
+// 4, 8 (within 16 lanes, by DPP: the mirrored orders pair the same partial sums),
+// 16 and 32: six VALU steps, where a shuffle through LDS took over 100 cycles each
+// (one request of 161 tokens, 43 LayerNorms in GEMM prologues: 734 -> 704 us).
+template <int STEP>
+__device__ inline float lane_pair_sum(float v) {
+    const int i = __builtin_bit_cast(int, v);
+    if constexpr (STEP < 16) {
+        constexpr int ctrl = STEP == 1 ? 0xB1 : STEP == 2 ? 0x4E : STEP == 4 ? 0x141 : 0x140;
+        return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, i, ctrl, 0xf, 0xf, true));
+    } else if constexpr (STEP == 16) {
+        const u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(i, i, false, false));
+        const uint32_t x = r[0], y = r[1];
+        return __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y);
+    } else {
+        const u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(i, i, false, false));
+        const uint32_t x = r[0], y = r[1];
+        return __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y);
+    }
 }
-// wave_sum of N values at once (the same steps for each), so their shuffles
-// share each LDS round trip.
+
+// Sums over the wavefront of N values at once, in every lane.
 template <int N>
 __device__ inline void wave_sum_n(float (&v)[N]) {
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
+    for (int r = 0; r < N; ++r) v[r] = lane_pair_sum<1>(v[r]);
 #pragma unroll
-        for (int r = 0; r < N; ++r) v[r] += __shfl_xor(v[r], o, JH_WAVE);
+    for (int r = 0; r < N; ++r) v[r] = lane_pair_sum<2>(v[r]);
+#pragma unroll
+    for (int r = 0; r < N; ++r) v[r] = lane_pair_sum<4>(v[r]);
+#pragma unroll
+    for (int r = 0; r < N; ++r) v[r] = lane_pair_sum<8>(v[r]);
+#pragma unroll
+    for (int r = 0; r < N; ++r) v[r] = lane_pair_sum<16>(v[r]);
+#pragma unroll
+    for (int r = 0; r < N; ++r) v[r] = lane_pair_sum<32>(v[r]);
 }
 
-__device__ inline float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, JH_WAVE));
-    return v;
+__device__ inline float wave_sum(float v) {
+    float s[1] = {v};
+    wave_sum_n(s);
+    return s[0];
 }
 
 // erf by the rational approximation published in Eigen (ptanh/perf float

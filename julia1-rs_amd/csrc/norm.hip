@@ -3,7 +3,7 @@
 // values per lane, loaded with the widest vector that divides them (float4
 // for hidden 768/1024, float2 for 384/128), so every global access is a fully
 // coalesced 64-lane vector load.  LayerNorm is two-pass (mean, then squared
-// deviations) with wavefront-shuffle sums, as in the reference's layer_norm.
+// deviations) with wavefront sums in registers, as in the reference's layer_norm.
 #include <hip/hip_runtime.h>
 
 #include "kernels.hpp"

@@ -2,7 +2,7 @@
 // hidden/64 values per lane, loaded with the widest vector that divides them
 // (float4 for hidden 768/1024, float2 for 384/128), so every global access is
 // a fully coalesced 64-lane vector load; and the two-pass LayerNorm over it
-// (mean, then squared deviations, with wavefront-shuffle sums).  Shared by the
+// (mean, then squared deviations, with wavefront sums in registers).  Shared by the
 // row kernels and the small-batch GEMM's LayerNorm prologue, so both produce
 // the same bits.
 #pragma once
