@@ -795,14 +795,45 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
     }
 }
 
+// What the elementwise epilogue of four features of row t (and of the four 32
+// above them) reads besides the sums: loaded ahead of them where that hides its
+// latency.
+struct FinishOps {
+    f32x4 bias[2], old[2], cos, sin;
+};
+
+// Bias and residual of features f .. f+3, operand h.
+template <int EPI>
+__device__ inline void load_finish(const GemmArgs& a, long t, int f, FinishOps& o, int h) {
+    const bool biased = EPI == JH_EPI_BIAS_BF16 || EPI == JH_EPI_BIAS_RELU_BF16 || EPI == JH_EPI_BIAS_F32 ||
+                        (EPI == JH_EPI_RESID_F32 && a.bias);
+    if (biased) o.bias[h] = *(const f32x4*)(a.bias + f);
+    if constexpr (EPI == JH_EPI_RESID_F32) o.old[h] = *(const f32x4*)((const float*)a.out + t * a.ldo + a.col + f);
+}
+
+// RoPE: row t's position, and with it the cos and sin of dims 4q .. +3.
+template <int EPI>
+__device__ inline uint32_t load_position(const GemmArgs& a, long t, int slab) {
+    return EPI == JH_EPI_ROPE_BF16 && slab < a.rope_cols ? (uint32_t)a.pos[t] & 0xffffu : 0u;
+}
+template <int EPI>
+__device__ inline void load_rope(const GemmArgs& a, uint32_t p, int slab, int q, FinishOps& o) {
+    if constexpr (EPI == JH_EPI_ROPE_BF16) {
+        if (slab < a.rope_cols) {
+            o.cos = *(const f32x4*)(a.cos_t + (long)p * 32 + 4 * q);
+            o.sin = *(const f32x4*)(a.sin_t + (long)p * 32 + 4 * q);
+        }
+    }
+}
+
 // Elementwise epilogue of FP32 sums for one output row t, features f .. f+3
 // (epilogues without a 64-feature pairing).
 template <int EPI>
-__device__ inline void finish_one(const GemmArgs& a, long t, int f, f32x4 v) {
+__device__ inline void finish_one(const GemmArgs& a, long t, int f, f32x4 v, const FinishOps& o, int h) {
     const bool biased = EPI == JH_EPI_BIAS_BF16 || EPI == JH_EPI_BIAS_RELU_BF16 || EPI == JH_EPI_BIAS_F32 ||
                         (EPI == JH_EPI_RESID_F32 && a.bias);
     if (biased) {
-        const f32x4 bb = *(const f32x4*)(a.bias + f);
+        const f32x4 bb = o.bias[h];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             v[e] += bb[e];
@@ -811,11 +842,10 @@ __device__ inline void finish_one(const GemmArgs& a, long t, int f, f32x4 v) {
     }
     const long c = a.col + f;
     if constexpr (EPI == JH_EPI_RESID_F32) {
-        float* o = (float*)a.out + t * a.ldo + c;
-        f32x4 r = *(const f32x4*)o;
+        f32x4 r = o.old[h];
 #pragma unroll
         for (int e = 0; e < 4; ++e) r[e] += v[e];
-        *(f32x4*)o = r;
+        *(f32x4*)((float*)a.out + t * a.ldo + c) = r;
     } else if constexpr (EPI == JH_EPI_BIAS_F32) {
         *(f32x4*)((float*)a.out + t * a.ldo + c) = v;
     } else {
@@ -827,15 +857,15 @@ __device__ inline void finish_one(const GemmArgs& a, long t, int f, f32x4 v) {
 // a 64-feature block: the RoPE pair (d, d+32) and the GEGLU pair (gate, up)
 // of an output are both here.
 template <int EPI>
-__device__ inline void finish_pair(const GemmArgs& a, long t, int slab, int q, f32x4 lo, f32x4 hi) {
+__device__ inline void finish_pair(const GemmArgs& a, long t, int slab, int q, f32x4 lo, f32x4 hi,
+                                   const FinishOps& o) {
     auto store_bf16 = [&](long col, f32x4 v) {
         *(u32x2*)((bf16_t*)a.out + t * a.ldo + col) = u32x2{pack2(v[0], v[1]), pack2(v[2], v[3])};
     };
     const long c0 = a.col + slab + 4 * q;
     if constexpr (EPI == JH_EPI_ROPE_BF16) {
         if (slab < a.rope_cols) {
-            const long ps = (long)(a.pos[t] & 0xffff) * 32 + 4 * q;
-            const f32x4 c = *(const f32x4*)(a.cos_t + ps), sn = *(const f32x4*)(a.sin_t + ps);
+            const f32x4 c = o.cos, sn = o.sin;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 float l = lo[e], h = hi[e];
@@ -852,8 +882,8 @@ __device__ inline void finish_pair(const GemmArgs& a, long t, int slab, int q, f
         for (int e = 0; e < 4; ++e) g[e] = gelu_erf(lo[e]) * hi[e];
         store_bf16(a.col + slab / 2 + 4 * q, g);
     } else {
-        finish_one<EPI>(a, t, slab + 4 * q, lo);
-        finish_one<EPI>(a, t, slab + 32 + 4 * q, hi);
+        finish_one<EPI>(a, t, slab + 4 * q, lo, o, 0);
+        finish_one<EPI>(a, t, slab + 32 + 4 * q, hi, o, 1);
     }
 }
 
@@ -872,11 +902,16 @@ __device__ inline void finish_pair(const GemmArgs& a, long t, int slab, int q, f
 // then apply the epilogue.
 //
 // LayerNorm prologue (LN_EPL > 0, hidden = 64 * LN_EPL = K): X comes from
-// FP32 rows.  Each wave loads its 8 rows after the first W segments are
-// issued, normalises them as layer_norm_kernel does (same code, same bits)
-// and writes the bf16 rows into the X segments; the first segment's barrier
-// publishes them.  This replaces a LayerNorm launch between a residual GEMM
-// and the next GEMM.
+// FP32 rows.  Each wave loads its 8 rows, then issues its share of all of W,
+// normalises the rows as layer_norm_kernel does (same code, same bits) while W
+// lands, and writes the bf16 rows into the X segments; one barrier publishes
+// both.  This replaces a LayerNorm launch between a residual GEMM and the next
+// GEMM.  (W first, the rows behind its first segments, and what the epilogue
+// reads loaded after the last MFMA: a request of 161 tokens took 704 us instead
+// of 670 at hidden 384.)
+//
+// At K = 384 the LDS is sized for two workgroups per CU (a request of 600 tokens
+// at hidden 384: 1077 -> 943 us).
 constexpr int SMALL_LDS = 96 * 768;  // bf16 elements of operand LDS per workgroup (144 KB)
 constexpr int SMALL_BT = 32;
 constexpr int SMALL_DEPTH = 6;  // K segments in flight ahead of the one being multiplied
@@ -922,7 +957,11 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(GemmArgs a) {
     constexpr int PW = (WI + XI) / 4;                  // ... per wave
     static_assert((WI + XI) % 4 == 0 && (BF == 64 || BF == 32), "tile shape");
     static_assert(!LNX || (BF == 64 && !GATHER), "LayerNorm prologue: 64-feature tiles, contiguous rows");
-    __shared__ __align__(1024) bf16_t smem[SMALL_LDS];
+    // The operands, and the four FP32 partial tiles afterwards.  With K known,
+    // no more than it needs: at K = 384 two workgroups then share a CU.
+    constexpr int LDS = CSEG ? std::max(CSEG * 64 * (BF + BT), 4 * BT * BF * 2) : SMALL_LDS;
+    static_assert(LDS <= SMALL_LDS, "operand LDS");
+    __shared__ __align__(1024) bf16_t smem[LDS];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nF = a.n / BF;
     const int f0 = (int)(blockIdx.x % nF) * BF, t0 = (int)(blockIdx.x / nF) * BT;
@@ -965,17 +1004,44 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(GemmArgs a) {
         }
     };
 
+    // The element this lane finishes: token 8 wave + lane/8, chunk q of the tile.
+    // What its epilogue reads (residual, bias, RoPE position) is loaded first of
+    // all, a round trip to memory that would otherwise follow the last MFMA.
+    const int tl = wave * 8 + (lane >> 3), q = lane & 7;
+    const long t = t0 + tl, tc = min(t, (long)a.rows - 1);
+    FinishOps fin;
+    load_finish<EPI>(a, tc, f0 + 4 * q, fin, 0);
+    if constexpr (BF == 64) load_finish<EPI>(a, tc, f0 + 32 + 4 * q, fin, 1);
+    const uint32_t fpos = load_position<EPI>(a, tc, f0);
+    __builtin_amdgcn_sched_barrier(0);
+
     int issued = min(SMALL_DEPTH, nseg);
-    for (int g = 0; g < issued; ++g) issue(g);
+    if constexpr (!LNX)
+        for (int g = 0; g < issued; ++g) issue(g);
     if constexpr (LNX) {
-        // Loads complete in issue order, so these rows arrive after the W
-        // segments issued above; the compiler's waits for them cover that.
+        // The rows first, so that they are normalised while W lands.  W goes
+        // by the builtin here: the compiler counts its operations, so a wait for
+        // the rows does not include them.
         constexpr int VEC = RowVec<LN_EPL>::VEC;
         RowVec<LN_EPL> xr[8], lw, lb;
 #pragma unroll
         for (int r = 0; r < 8; ++r) xr[r].load(a.xf + (long)min(t0 + wave * 8 + r, a.rows - 1) * a.ldx, lane);
         lw.load(a.ln_w, lane);
         if (a.ln_b) lb.load(a.ln_b, lane);
+        __builtin_amdgcn_sched_barrier(0);
+        const __amdgpu_buffer_rsrc_t bw =
+            __builtin_amdgcn_make_buffer_rsrc((void*)(a.w + (long)f0 * a.k), 0, (int)(BF * a.k * 2), 0x00020000);
+        typedef __attribute__((address_space(3))) void lds_void;
+#pragma unroll
+        for (int g = 0; g < CSEG; ++g)
+#pragma unroll
+            for (int u = 0; u < PW; ++u) {
+                const int j = wave * PW + u, row = j * 8 + (lane >> 3);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(bw, (lds_void*)&sW[(g * BF + j * 8) * 64], 16,
+                                                         (int)(row * a.k + (((lane & 7) ^ swz(row)) * 8)) * 2, g * 128, 0, 0);
+            }
+        load_rope<EPI>(a, fpos, f0, q, fin);
+        __builtin_amdgcn_sched_barrier(0);
         // RowVec::layer_norm's steps with the 8 rows' reductions interleaved.
         float st[8], mean[8];
 #pragma unroll
@@ -1018,7 +1084,12 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(GemmArgs a) {
             acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, bx, acc[i], 0, 0, 0);
         }
     };
-    if constexpr (CSEG > 0) {
+    if constexpr (LNX) {
+        vmcnt<0>();
+        __syncthreads();
+#pragma unroll
+        for (int g = 0; g < CSEG; ++g) multiply(g);
+    } else if constexpr (CSEG > 0) {
         constexpr int NSEG = CSEG, ISSUED0 = NSEG < SMALL_DEPTH ? NSEG : SMALL_DEPTH;
         [&]<int... G>(std::integer_sequence<int, G...>) {
             (
@@ -1055,9 +1126,7 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(GemmArgs a) {
             *(f32x4*)&red[slot(wave, lr, i * 8 + qd * 2 + lg)] = v;
         }
     __syncthreads();
-    // Wave w finishes tokens 8w .. 8w+7, lane -> (token 8w + lane/8, chunk q).
-    const int tl = wave * 8 + (lane >> 3), q = lane & 7;
-    const long t = t0 + tl;
+    // Wave w finishes tokens 8w .. 8w+7.
     if (t >= a.rows) return;
     auto total = [&](int ch) {
         f32x4 s = *(const f32x4*)&red[slot(0, tl, ch)];
@@ -1069,8 +1138,9 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(GemmArgs a) {
         }
         return s;
     };
-    if constexpr (BF == 64) finish_pair<EPI>(a, t, f0, q, total(q), total(q + 8));
-    else finish_one<EPI>(a, t, f0 + 4 * q, total(q));
+    if constexpr (!LNX) load_rope<EPI>(a, fpos, f0, q, fin);
+    if constexpr (BF == 64) finish_pair<EPI>(a, t, f0, q, total(q), total(q + 8), fin);
+    else finish_one<EPI>(a, t, f0 + 4 * q, total(q), fin, 0);
 }
 
 // Split-K reduction + epilogue: thread (row t, 64-wide slab, q) sums the S
@@ -1103,7 +1173,11 @@ __global__ __launch_bounds__(256) void splitk_reduce(GemmArgs a, int S) {
             lo[e] = s < S ? lo[e] + pl[s][e] : lo[e];
             hi[e] = s < S ? hi[e] + ph[s][e] : hi[e];
         }
-    finish_pair<EPI>(a, t, slab, q, lo, hi);
+    FinishOps o;
+    load_finish<EPI>(a, t, slab + 4 * q, o, 0);
+    load_finish<EPI>(a, t, slab + 32 + 4 * q, o, 1);
+    load_rope<EPI>(a, load_position<EPI>(a, t, slab), slab, q, o);
+    finish_pair<EPI>(a, t, slab, q, lo, hi, o);
 }
 
 // Tile shape: 128 features x 128 tokens, four waves of 64x64, two resident
@@ -1171,14 +1245,14 @@ int small_bf(int epi, const GemmArgs& a) {
 // Waves per workgroup of the slab-resident kernel (K = 384) for `a`, or 0 when
 // launch_gemm does not use it.  It sums K in steps of 32, the tiled kernels in
 // steps of 16, so like the small-batch paths it is left out when a row must not
-// depend on the batch (no workspace).  Measured (us, tiled or small-batch kernel
+// depend on the batch (no workspace).  Measured (us, small-batch or tiled kernel
 // against this one), by N and tokens:
-//   N = 384: 933 4.2 / 5.3, 1500 7.1 / 6.7, 3300 10.6 / 7.4, 4323 13.2 / 7.9,
-//     7556 10.6 / 10.2, 16384 14.5 / 13.7, 65536 58.8 / 55.6: from the second
-//     round of the small-batch kernel's 64 x 32 tiles on (one per CU);
-//   N = 1152: 600 6.7 / 7.3, 933 8.8 / 7.6, 1500 12.0 / 7.8, 2500 9.5 / 9.8,
-//     4323 12.2 / 12.7; N = 2304: 400 6.4 / 7.7, 600 8.7 / 7.9, 1500 8.3 / 9.6:
-//     from the small-batch kernel's third round to its last;
+//   N = 384: 933 4.0 / 5.3, 1500 4.9 / 6.8, 2500 5.8 / 6.5, 3000 6.8 / 6.5, 4323
+//     9.7 / 7.8, 7556 10.6 / 10.2, 16384 14.5 / 13.7, 65536 58.8 / 55.6: from the
+//     second round of the small-batch kernel's 64 x 32 tiles on (two per CU);
+//   N = 1152: 1200 6.7 / 7.0, 1500 8.3 / 6.8, 2500 9.5 / 9.8, 4323 12.2 / 12.7;
+//   N = 2304: 600 6.6 / 6.8, 700 7.2 / 6.7, 800 7.4 / 7.1, 1500 8.3 / 9.6: from one
+//     and a half rounds to the small-batch kernel's last size;
 //   twelve waves (384-row slabs), N = 1152: 9500 15.5 / 17.7, 16384 24.0 / 24.0,
 //     65536 96 / 66; N = 2304: 16384 38.9 / 37.1, 65536 167 / 124.
 int slab_waves(const GemmArgs& a) {
@@ -1186,8 +1260,8 @@ int slab_waves(const GemmArgs& a) {
     if (a.rows >= 16384 && a.n >= 1024 && a.n % 384 == 0) return 12;
     const long cus = resident_tiles() / 2, tiles = (long)((a.n + 127) / 128) * ((a.rows + 127) / 128);
     const long small = (long)(a.n / 64) * ((a.rows + SMALL_BT - 1) / SMALL_BT);
-    if (a.n < 1024) return small > cus ? 4 : 0;
-    return tiles < 128 && small > 2 * cus ? 4 : 0;
+    if (a.n < 1024) return small > 2 * cus ? 4 : 0;
+    return tiles < 128 && small > 3 * cus ? 4 : 0;
 }
 
 // Whether launch_gemm runs `a` on the weight-stationary kernel (K = 768, or 1152

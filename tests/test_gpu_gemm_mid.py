@@ -51,9 +51,9 @@ def _out(rows, width, epi, col, pad, seed):
     return torch.randn(rows + 1, col + width + pad, generator=g, device="cuda").to(torch.float32 if f32 else BF16)
 
 
-# (rows, n): the first two are each one row past the small-batch kernel's last size; 16-token units at
-# 16384 + 1; a 128-row slab count that is no multiple of three
-SLAB = [(1361, 384), (705, 1152), (929, 1152), (1792, 1152), (2049, 256), (4323, 384), (16384, 1152), (16385, 2304),
+# (rows, n): the first ones each one row past (or at) the small-batch kernel's last size and the rule's end; then a
+# 128-row slab count that is no multiple of three, and 384-row slabs from 16384 rows on
+SLAB = [(2721, 384), (1345, 1152), (1792, 1152), (673, 2304), (4097, 256), (4323, 384), (16384, 1152), (16385, 2304),
         (20003, 1536)]
 
 
