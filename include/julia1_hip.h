@@ -190,8 +190,8 @@ int jh_set_graph(jh_model* model, int enabled);
  * too few 128 x 128 tiles to occupy the GPU (small batches, marker rows), K is
  * split: over the four waves of one workgroup (one launch, K <= 768) or into
  * chunks whose FP32 partial sums a second kernel reduces (the residual GEMMs,
- * with the residual add and LayerNorm in that kernel).  Full attention over
- * few, long rows likewise splits the keys of a query over groups of waves.
+ * with the residual add and LayerNorm in that kernel).  Attention over few
+ * rows likewise splits the keys of a query over groups of waves.
  * Either way the partial
  * sums are added in a fixed order, so results are deterministic, but a row's
  * FP32 summation order then depends on the batch's token count.  Off, every output element is accumulated in the same

@@ -190,9 +190,9 @@ typedef struct jh_attn_tile {
  * q/k/v bf16 with row strides ldq/ldkv; head h reads columns [64h, 64h+64)
  * of each; out bf16 row stride ldo.  `tiles` is a device array; work items
  * are dispatched in list order with heads varying fastest, so listing the
- * costliest tiles first (as the backend does) balances the CUs.  Full
- * attention with few work items (at most two per CU) over long rows splits
- * each item's keys over two or four groups of waves, which adds a query's
+ * costliest tiles first (as the backend does) balances the CUs.  Few work
+ * items (at most one for every two CUs, or two per CU over long rows) have
+ * their keys split over two or four groups of waves, which adds a query's
  * partial sums in another order.
  * Replaces attention_rope/attention_plain (src/cuda/kernels.cu:274-391); RoPE
  * is applied by the producing GEMM's ROPE epilogue instead of on every load.

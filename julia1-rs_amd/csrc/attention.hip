@@ -71,20 +71,24 @@ __device__ constexpr int vswz(int r) { return ((r >> 1) & 1) << 2; }
 // eight-wave form stages two key tiles per barrier (four 16 KB K/V slots,
 // 64 KB: two workgroups per CU still fit), which halves the barriers each
 // wave meets (a further 1.8% at 4 x 8192).
-// KS > 1 splits the keys of a 128-query item over KS groups of four waves: a
-// stage holds KS key tiles, group g runs tile g of each, and at the end the
-// groups' running maxima, sums and outputs are merged through LDS in group order.
+// KS > 1 splits the keys over KS groups of QG = NW / KS waves: a stage holds KS
+// key tiles, group g runs tile g of each, and at the end the groups' running
+// maxima, sums and outputs are merged through LDS in group order.
+template <int NW, int KS>
+constexpr int stage_tiles() {  // key tiles staged per barrier
+    return KS > 1 ? KS : NW / 4;
+}
 template <int NW, bool WIN, int KS>  // WIN: a window layer (a.window >= 0), whose tiles run one 32-key block per step
 __device__ __forceinline__ void attend(const AttnArgs& a, const AttnTile& tile, const int head,
-                                       bf16_t (&smem)[2][NW / 2][KT * 64]) {
-    static_assert(KS == 1 || NW == 4 * KS, "key-split items have 128 queries");
-    constexpr int SPB = NW / 4;           // key tiles staged per barrier
+                                       bf16_t (&smem)[2][2 * stage_tiles<NW, KS>()][KT * 64]) {
+    constexpr int SPB = stage_tiles<NW, KS>();
     constexpr int RPW = SPB * KT / NW;    // K/V rows each wave stages per barrier (8 per DMA instruction)
+    constexpr int QG = NW / KS;           // query groups of 32
     auto& sK = smem[0];
     auto& sV = smem[1];
     const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wave = KS > 1 ? wid & 3 : wid;  // query group of the wave
-    const int kgrp = KS > 1 ? wid >> 2 : 0;   // key group of the wave
+    const int wave = wid % QG;  // query group of the wave
+    const int kgrp = wid / QG;  // key group of the wave
     const int lq = lane & 31, g = lane >> 5;
 
     const bf16_t* kbase = a.k + (long)tile.kv_row * a.ldkv + head * 64;
@@ -112,6 +116,8 @@ __device__ __forceinline__ void attend(const AttnArgs& a, const AttnTile& tile, 
     int kbeg = 0, kend = tile.kv_len;
     if (a.window >= 0) {
         kbeg = max(0, tile.q_pos - a.window);
+        // (the same tiles, in the same groups, for the sub-items of any size)
+        if (KS > 1) kbeg &= ~(KT - 1);
         kend = min(tile.kv_len, tile.q_pos + tile.nq + a.window);
     }
 
@@ -138,6 +144,7 @@ __device__ __forceinline__ void attend(const AttnArgs& a, const AttnTile& tile, 
 #pragma unroll
         for (int j = 0; j < RPW / 8; ++j) {
             const int r0 = RPW * wid + 8 * j;
+            if (KS > 1 && k0 + (r0 & ~(KT - 1)) >= kend) continue;  // (no such tile)
             const uint32_t lk = __builtin_amdgcn_readfirstlane(lk0 + (st * SPB * KT * 64 + r0 * 64) * 2);
             const uint32_t lv = __builtin_amdgcn_readfirstlane(lv0 + (st * SPB * KT * 64 + r0 * 64) * 2);
             asm volatile("buffer_load_dwordx4 %1, %2, 0 offen lds" ::"{m0}"(lk), "v"(okb[j] + kt), "s"(rsk)
@@ -338,25 +345,27 @@ __device__ __forceinline__ void attend(const AttnArgs& a, const AttnTile& tile, 
     }
 
     if constexpr (KS > 1) {
-        // Merge in group order.  A group that saw no key of a query has m = -inf,
-        // l = 0 and o = 0, and weighs nothing.
+        // Merge in group order, as many groups as had a tile.  A group that saw no
+        // key of a query has m = -inf, l = 0 and o = 0, and weighs nothing.
         float* const part = (float*)smem;  // [group 1 ..][wave][34][lane]
-        __syncthreads();  // every wave is done with the K/V tiles
-        if (kgrp > 0) {
-            float* p = part + ((kgrp - 1) * 4 + wave) * 34 * 64 + lane;
+        const int groups = min(KS, ntk);
+        if (groups > 1) {
+            __syncthreads();  // every wave is done with the K/V tiles
+            if (kgrp > 0 && kgrp < groups) {
+                float* p = part + ((kgrp - 1) * QG + wave) * 34 * 64 + lane;
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                p[e * 64] = o[0][e];
-                p[(16 + e) * 64] = o[1][e];
+                for (int e = 0; e < 16; ++e) {
+                    p[e * 64] = o[0][e];
+                    p[(16 + e) * 64] = o[1][e];
+                }
+                p[32 * 64] = m;
+                p[33 * 64] = l;
             }
-            p[32 * 64] = m;
-            p[33 * 64] = l;
+            __syncthreads();
         }
-        __syncthreads();
         if (kgrp > 0) return;
-#pragma unroll
-        for (int g2 = 0; g2 < KS - 1; ++g2) {
-            const float* p = part + (g2 * 4 + wave) * 34 * 64 + lane;
+        for (int g2 = 0; g2 < groups - 1; ++g2) {
+            const float* p = part + (g2 * QG + wave) * 34 * 64 + lane;
             const float m2 = p[32 * 64], mn = fmaxf(m, m2);
             const float w1 = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m - mn) * c);
             const float w2 = m2 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m2 - mn) * c);
@@ -384,30 +393,32 @@ __device__ __forceinline__ void attend(const AttnArgs& a, const AttnTile& tile, 
     }
 }
 
-// KS > 1: items whose keys are too few for the split to pay (a caller that knows
-// of none as long says so in key_split) run as with KS = 1, on the first four waves.  Measured (us,
+// 128-query items, KS > 1: those whose keys are too few for the split to pay (where
+// the caller does not say so in a.longest, the launch knows only their number) run as with KS = 1, on the first four waves.  Measured (us,
 // hidden 384, one row of 500 / 900 / 1500 / 3928 keys): KS 1 10.0 / 15.1 / 22.0
 // / 50.4, KS 4 10.9 / 14.3 / 18.6 / 39.0; KS 2 at two items per CU: 8 rows of
 // 900 keys 23.6 -> 23.9, 4 of 1500 31.4 -> 30.3, one of 8192 138 -> 129.
-constexpr int kSplitKeys4 = ATTN_SPLIT_KEYS, kSplitKeys2 = 1152;
+constexpr int kSplitKeys4 = 832, kSplitKeys2 = 1152;
 
-// HALVES: two workgroups per 256-query tile, each with 128 of its queries.
-template <int NW, bool WIN, int KS = 1, bool HALVES = false>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(4))) void attention_kernel(AttnArgs a) {
-    __shared__ __align__(1024) bf16_t smem[2][NW / 2][KT * 64];
+// SUB workgroups share a tile of the list, each with 32 NW / KS of its queries.
+template <int NW, bool WIN, int KS = 1, int SUB = 1>
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(KS == 4 ? NW / 4 : 4))) void attention_kernel(
+    AttnArgs a) {
+    constexpr int SUBQ = 32 * NW / KS;
+    __shared__ __align__(1024) bf16_t smem[2][2 * stage_tiles<NW, KS>()][KT * 64];
     // One workgroup per (tile, head), heads varying fastest: callers list the
     // costliest tiles first, so those are dispatched first, one per CU.
     const int head = (int)(blockIdx.x % (unsigned)a.heads);
     const int item = (int)(blockIdx.x / (unsigned)a.heads);
-    AttnTile tile = a.tiles[HALVES ? item >> 1 : item];
-    if constexpr (HALVES) {
-        const int off = (item & 1) * 128;
+    AttnTile tile = a.tiles[item / SUB];
+    if constexpr (SUB > 1) {
+        const int off = item % SUB * SUBQ;
         if (off >= tile.nq) return;
         tile.q_row += off;
         tile.q_pos += off;
-        tile.nq = min(tile.nq - off, 128);
+        tile.nq = min(tile.nq - off, SUBQ);
     }
-    if constexpr (KS > 1) {
+    if constexpr (KS > 1 && SUBQ == 128) {
         if (tile.kv_len < (KS == 4 ? kSplitKeys4 : kSplitKeys2)) {
             if (threadIdx.x >= 256) return;
             attend<4, WIN, 1>(a, tile, head, *(bf16_t(*)[2][2][KT * 64])smem);
@@ -434,12 +445,38 @@ double halves_cost(long items, long cus) {
     return full * 2.06 + (rest == 0 ? 0.0 : rest <= cus ? 0.75 : rest <= 2 * cus ? 1.17 : rest <= 3 * cus ? 1.75 : 2.06);
 }
 
-template <bool HALVES>
-void launch_items(const AttnArgs& a, int ks, dim3 grid, hipStream_t s) {
-    if (ks == 4) JH_LAUNCH((attention_kernel<16, false, 4, HALVES>), grid, dim3(1024), 0, s, a);
-    else if (ks == 2) JH_LAUNCH((attention_kernel<8, false, 2, HALVES>), grid, dim3(512), 0, s, a);
-    else if (a.window >= 0) JH_LAUNCH((attention_kernel<4, true, 1, HALVES>), grid, dim3(256), 0, s, a);
-    else JH_LAUNCH((attention_kernel<4, false, 1, HALVES>), grid, dim3(256), 0, s, a);
+// The 128-query items of the list's tiles, TQ / 128 to a tile.
+template <int TQ>
+void launch_items(const AttnArgs& a, hipStream_t s) {
+    const long cus = gemm_resident_tiles() / 2, items = (long)a.ntiles * a.heads * (TQ / 128);
+    auto grid = [&](int sub) { return dim3((unsigned)((long)a.ntiles * a.heads * sub)); };
+    const bool win = a.window >= 0;
+    // Few items leave SIMDs with one or two waves, or none.  The keys of each are
+    // then split four (two) ways, and where the items are few for the CUs its
+    // queries over two or four workgroups too.  Not for rows of one key tile; the
+    // unsplit queries only over long rows (see kSplitKeys4), and not on window
+    // layers, whose items have at most four or five key tiles.  Measured (us, one
+    // row, hidden 384, full attention, 128-query items / four ways / and 64-query
+    // workgroups): 500 keys 9.9 / 10.9 / 8.0, 933 15.1 / 14.4 / 10.6, 1500 22.0 / 18.7
+    // / 13.8, 2500 34.4 / 26.7 / 20.4; a whole request, 128-query items / 64 / 32: 161
+    // tokens 671 / 666 / 659, 300 763 / 741 / 736, 1200 1177 / 1121 / 1125; 30 tokens
+    // 603 / 614 / 622.
+    const bool split = a.key_split && (!a.longest || a.longest > KT);
+    if (split && 8 * items <= cus) {
+        if (win) JH_LAUNCH((attention_kernel<4, true, 4, TQ / 32>), grid(TQ / 32), dim3(256), 0, s, a);
+        else JH_LAUNCH((attention_kernel<4, false, 4, TQ / 32>), grid(TQ / 32), dim3(256), 0, s, a);
+    } else if (split && 2 * items <= cus) {
+        if (win) JH_LAUNCH((attention_kernel<8, true, 4, TQ / 64>), grid(TQ / 64), dim3(512), 0, s, a);
+        else JH_LAUNCH((attention_kernel<8, false, 4, TQ / 64>), grid(TQ / 64), dim3(512), 0, s, a);
+    } else if (split && !win && items <= cus && (!a.longest || a.longest >= kSplitKeys4)) {
+        JH_LAUNCH((attention_kernel<16, false, 4, TQ / 128>), grid(TQ / 128), dim3(1024), 0, s, a);
+    } else if (split && !win && items > cus && items <= 2 * cus && (!a.longest || a.longest >= kSplitKeys2)) {
+        JH_LAUNCH((attention_kernel<8, false, 2, TQ / 128>), grid(TQ / 128), dim3(512), 0, s, a);
+    } else if (win) {
+        JH_LAUNCH((attention_kernel<4, true, 1, TQ / 128>), grid(TQ / 128), dim3(256), 0, s, a);
+    } else {
+        JH_LAUNCH((attention_kernel<4, false, 1, TQ / 128>), grid(TQ / 128), dim3(256), 0, s, a);
+    }
 }
 
 }  // namespace
@@ -452,22 +489,10 @@ void launch_attention(const AttnArgs& a, hipStream_t s) {
     if (a.ldq % 8 || a.ldkv % 8 || a.ldo % 4 || a.ldq < a.heads * 64 || a.ldo < a.heads * 64 ||
         ((uintptr_t)a.q & 15) || ((uintptr_t)a.k & 15) || ((uintptr_t)a.v & 15) || ((uintptr_t)a.out & 7))
         throw jh_error(1, "attention: operands must be 16-byte aligned with row strides % 8 == 0");
-    if ((long)a.ntiles * a.heads > 0x3fffffffL) throw jh_error(1, "attention: grid too large");
-    const long cus = gemm_resident_tiles() / 2;
-    long items = (long)a.ntiles * a.heads;
-    bool wide = a.waves == 8, halves = false;
-    if (wide && (a.window >= 0 || halves_cost(items, cus) < wide_cost(items, cus))) {
-        halves = true;
-        wide = false;
-        items *= 2;
-    }
-    // Few items leave SIMDs with one or two waves, or none: full attention over
-    // long rows then splits each item's keys over two or four times the waves.
-    // (Not window layers: an item has at most four or five key tiles.)
-    const int ks = wide || !a.key_split || a.window >= 0 ? 1 : items <= cus ? 4 : items <= 2 * cus ? 2 : 1;
-    const dim3 grid((unsigned)items);
-    if (wide) JH_LAUNCH((attention_kernel<8, false>), grid, dim3(512), 0, s, a);
-    else if (halves) launch_items<true>(a, ks, grid, s);
-    else launch_items<false>(a, ks, grid, s);
+    if ((long)a.ntiles * a.heads > 0x0fffffffL) throw jh_error(1, "attention: grid too large");
+    const long cus = gemm_resident_tiles() / 2, items = (long)a.ntiles * a.heads;
+    if (a.waves == 4) launch_items<128>(a, s);
+    else if (a.window >= 0 || halves_cost(items, cus) < wide_cost(items, cus)) launch_items<256>(a, s);
+    else JH_LAUNCH((attention_kernel<8, false>), dim3((unsigned)items), dim3(512), 0, s, a);
     HIP_CHECK(hipGetLastError());
 }

@@ -165,9 +165,9 @@ struct MetaSlot {
     size_t markers = 0;
     // graph of the launch sequence for the shape staged in this slot
     hipGraphExec_t graph = nullptr;
-    size_t graph_key[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    size_t graph_key[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     // shape of the previous execute from this slot: captured only when it repeats
-    size_t last_key[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    size_t last_key[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
 };
 
 }  // namespace
@@ -527,7 +527,11 @@ struct jh_model {
                    long ldo, const AttnTile* tiles, size_t n, int nheads, int window, double pairs, double qrows,
                    int waves = 4) {
         AttnArgs a{q, ldq, k, v, ldkv, out, ldo, tiles, (int)n, nheads, window, 0.125f * 1.4426950408889634f, waves};
-        a.key_split = use_splitk && longest >= (uint32_t)ATTN_SPLIT_KEYS;
+        // Up to 512 tokens the splits gain 1.5 to 3.5% of a request, but a row alone
+        // would then differ in every attention layer from the same row in a larger
+        // batch: logits moved by up to 2.1e-3, past the 2e-3 that split-K keeps to.
+        a.key_split = use_splitk && longest > 512;
+        a.longest = (int)longest;
         const double hd = 64.0 * nheads;
         timed(cls, 4.0 * hd * pairs, qrows * hd * 2 * 2 + (double)T * hd * 2 * 2, [&] { launch_attention(a, stream); });
         if (profiling && !replay[cls]) replay[cls] = [a, st = stream] { launch_attention(a, st); };
@@ -679,15 +683,14 @@ struct jh_model {
             return;
         }
         MetaSlot& ms = slots[cur];
-        const size_t key[8] = {T, M, S, ntiles, nmtiles, (size_t)ws_gen, nglong,
-                               2 * ngshort + (longest >= (uint32_t)ATTN_SPLIT_KEYS)};
-        if (!ms.graph || !std::equal(key, key + 8, ms.graph_key)) {
+        const size_t key[9] = {T, M, S, ntiles, nmtiles, (size_t)ws_gen, nglong, ngshort, longest};
+        if (!ms.graph || !std::equal(key, key + 9, ms.graph_key)) {
             // Capturing and instantiating the ~200-launch forward costs ~0.5 ms
             // on MI355X while replay saves nothing measurable over eager
             // launches, so a shape seen for the first time in a row runs
             // eagerly; the graph is built when the same shape comes again.
-            if (!std::equal(key, key + 8, ms.last_key)) {
-                std::copy(key, key + 8, ms.last_key);
+            if (!std::equal(key, key + 9, ms.last_key)) {
+                std::copy(key, key + 9, ms.last_key);
                 run_all();
                 return;
             }
@@ -714,7 +717,7 @@ struct jh_model {
                 ms.graph = nullptr;
                 throw jh_error(JH_ERR_DEVICE, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
             }
-            std::copy(key, key + 8, ms.graph_key);
+            std::copy(key, key + 9, ms.graph_key);
         }
         HIP_CHECK(hipGraphLaunch(ms.graph, stream));
     }

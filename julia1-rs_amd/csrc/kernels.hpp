@@ -114,9 +114,9 @@ struct AttnArgs {
     int window;        // < 0: global
     float scale_log2;  // softmax scale · log2(e)
     int waves = 4;     // waves per work item: 4 (tiles of <= 128 queries) or 8 (<= 256 queries)
-    bool key_split = true;  // few items with ATTN_SPLIT_KEYS keys or more may share a query's keys among several waves
+    bool key_split = true;  // few items may share the keys of a query among several waves
+    int longest = 0;        // keys of the longest tile (0: not known)
 };
-constexpr int ATTN_SPLIT_KEYS = 832;
 
 void launch_attention(const AttnArgs& a, hipStream_t stream);
 

@@ -715,16 +715,21 @@ def test_attention_full_length_8192(window):
 
 
 @pytest.mark.parametrize("rate", [0.0, 0.4])
+@pytest.mark.parametrize("window", [-1, 64, 8])
 @pytest.mark.parametrize("heads,lens,wide", [
-    (2, [831, 832, 833, 960, 1], False),   # at most one item per CU: keys split four ways from 832 on
+    (2, [30, 161, 64, 65, 129], False),    # at most 32 items: 32-query workgroups, keys split four ways
+    (2, [831, 832, 300, 960, 1], False),   # at most 128: 64-query workgroups
+    (6, [831, 832, 833, 1], False),        # at most one 128-query item per CU: split from 832 keys on
     (12, [1151, 1152, 1153, 130], False),  # up to two per CU: two ways from 1152 on
     (12, [1407, 1300], True),              # 256-query tiles run as two 128-query workgroups each
+    (2, [300, 257], True),                 # ... and as eight of 32 queries
 ])
-def test_attention_key_split(heads, lens, wide, rate):
-    """Few work items over long rows: groups of waves take every second or fourth key tile and merge their running
-    maxima, sums and outputs.  With `rate`, scores climb along the row (log2 units per key tile), so the groups'
-    maxima differ and a group may hold almost all of the weight.  Each output is a weighted mean of v with P and
-    the result rounded to bf16 (2^-9 each) and scores summed in FP32, so its error is within 2^-8 max|v|."""
+def test_attention_key_split(heads, lens, wide, window, rate):
+    """Few work items: groups of waves take every second or fourth key tile and merge their running maxima, sums and
+    outputs, over fewer queries each where the items are very few.  With `rate`, scores climb along the row (log2
+    units per key tile), so the groups' maxima differ and a group may hold almost all of the weight.  Each output is
+    a weighted mean of v with P and the result rounded to bf16 (2^-9 each) and scores summed in FP32, so its error is
+    within 2^-8 max|v|."""
     r = rng(57)
     h = heads * 64
     t = sum(lens)
@@ -738,11 +743,11 @@ def test_attention_key_split(heads, lens, wide, rate):
         seqs.append((start, ln, start, ln, 0))
         start += ln
     qkv = bf16_round(np.concatenate([q, k, v], 1).astype(np.float32))
-    expect = _attn_ref64(qkv[:, :h], qkv[:, h:2 * h], qkv[:, 2 * h:], seqs, heads, -1)
+    expect = _attn_ref64(qkv[:, :h], qkv[:, h:2 * h], qkv[:, 2 * h:], seqs, heads, window)
     dq = dev(qkv, BF16)
     out = torch.zeros(t, h, dtype=BF16, device="cuda")
     hip.op_attention(dq, 3 * h, dq[:, h:], dq[:, 2 * h:], 3 * h, out, h,
-                     dev(np.array(_tiles(lens, 256 if wide else 128), dtype=np.int32)), heads, -1, wide=wide)
+                     dev(np.array(_tiles(lens, 256 if wide else 128), dtype=np.int32)), heads, window, wide=wide)
     assert np.abs(qkv[:, 2 * h:]).max() < 5.5
     assert np.abs(host(out) - expect).max() < 2.0 ** -8 * 5.5, np.abs(host(out) - expect).max()
 
