@@ -63,6 +63,24 @@ __device__ inline i32x4 make_rsrc(const void* base, uint64_t bytes) {
                  (int)(uint32_t)(bytes < 0xffffffffull ? bytes : 0xffffffffull), 0x00020000};
 }
 
+// Work item of workgroup b of G, item numbers in contiguous runs per XCD (workgroup
+// b runs on XCD b % 8).
+__device__ inline int xcd_run(int b, int G) {
+    const int xcd = b & 7, q8 = G >> 3, r8 = G & 7;
+    return xcd * q8 + (xcd < r8 ? xcd : r8) + (b >> 3);
+}
+
+// Item (slab or feature tile f of nF, token range r of nR) of a GEMM's workgroup.
+// An XCD's L2 holds what its own workgroups fetch: with items in token order it
+// fetches its eighth of X and all of W, in slab order its eighth of W and all of X.
+// Slab order is taken where W is the larger, N > tokens.
+__device__ inline void xcd_item(int b, int nF, int nR, bool slab_order, int& f, int& r) {
+    const int u = xcd_run(b, nF * nR);
+    const int d = slab_order ? nR : nF, hi = u / d, lo = u - hi * d;
+    f = slab_order ? hi : lo;
+    r = slab_order ? lo : hi;
+}
+
 // v plus the same value of another lane, lanes paired as in a butterfly over 1, 2,
 // 4, 8 (within 16 lanes, by DPP: the mirrored orders pair the same partial sums),
 // 16 and 32: six VALU steps, where a shuffle through LDS took over 100 cycles each

@@ -964,7 +964,9 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(GemmArgs a) {
     __shared__ __align__(1024) bf16_t smem[LDS];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nF = a.n / BF;
-    const int f0 = (int)(blockIdx.x % nF) * BF, t0 = (int)(blockIdx.x / nF) * BT;
+    int f, r;
+    xcd_item((int)blockIdx.x, nF, (a.rows + BT - 1) / BT, a.n > a.rows, f, r);
+    const int f0 = f * BF, t0 = r * BT;
     const int nseg = CSEG ? CSEG : a.k / 64;  // 128-byte row segments
     bf16_t* const sW = smem;                   // segment g: rows [0, BF) at sW + g*BF*64
     bf16_t* const sX = smem + nseg * BF * 64;  // segment g: rows [0, BT) at sX + g*BT*64
@@ -1242,6 +1244,12 @@ int small_bf(int epi, const GemmArgs& a) {
     return a.k <= small_kmax<64>() ? 64 : 0;
 }
 
+// Row strides with which the slab-resident and weight-stationary kernels may stand
+// in for the small-batch and split-K ones: they address 16 rows of X and of the
+// output with 32-bit byte offsets (16 * 2^24 floats are 2^30 bytes), the others the
+// output with 64-bit addresses.
+bool narrow_strides(const GemmArgs& a) { return a.ldx <= 1L << 24 && a.ldo <= 1L << 24; }
+
 // Waves per workgroup of the slab-resident kernel (K = 384) for `a`, or 0 when
 // launch_gemm does not use it.  It sums K in steps of 32, the tiled kernels in
 // steps of 16, so like the small-batch paths it is left out when a row must not
@@ -1256,7 +1264,7 @@ int small_bf(int epi, const GemmArgs& a) {
 //   twelve waves (384-row slabs), N = 1152: 9500 15.5 / 17.7, 16384 24.0 / 24.0,
 //     65536 96 / 66; N = 2304: 16384 38.9 / 37.1, 65536 167 / 124.
 int slab_waves(const GemmArgs& a) {
-    if (!a.partial || a.splits != 0 || !gemm_slab_supported(a)) return 0;
+    if (!a.partial || a.splits != 0 || !gemm_slab_supported(a) || !narrow_strides(a)) return 0;
     if (a.rows >= 16384 && a.n >= 1024 && a.n % 384 == 0) return 12;
     const long cus = resident_tiles() / 2, tiles = (long)((a.n + 127) / 128) * ((a.rows + 127) / 128);
     const long small = (long)(a.n / 64) * ((a.rows + SMALL_BT - 1) / SMALL_BT);
@@ -1284,7 +1292,7 @@ int slab_waves(const GemmArgs& a) {
 // 30.8 / 27.5; K = 1152, N = 768: 7556 22.4 / 19.8, 16384 45.6 / 47.2.
 bool ws_takes(int epi, const GemmArgs& a) {
     if (!a.partial) return gemm_ws_supported(epi, a);
-    if (!gemm_ws_shape(epi, a) || (a.w_ws && !gemm_ws_supported(epi, a))) return false;
+    if (!gemm_ws_shape(epi, a) || (a.w_ws && !gemm_ws_supported(epi, a)) || !narrow_strides(a)) return false;
     const long cus = resident_tiles() / 2, tiles = (long)((a.n + 127) / 128) * ((a.rows + 127) / 128);
     const long small = (long)(a.n / (a.k <= small_kmax<64>() ? 64 : 32)) * ((a.rows + SMALL_BT - 1) / SMALL_BT);
     if (a.w_ws) return a.n < 1024 || a.k > small_kmax<64>() ? small > cus : 4 * small > 5 * cus;

@@ -134,12 +134,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    // Workgroup -> (token range r, slab f): consecutive ids u share r, and an
-    // XCD (workgroup b runs on XCD b % 8) gets a contiguous run of u.
-    const int G = gridDim.x, bid = blockIdx.x;
-    const int xcd = bid & 7, local = bid >> 3, q8 = G >> 3, r8 = G & 7;
-    const int u = xcd * q8 + (xcd < r8 ? xcd : r8) + local;
-    const int r = u / nF, f = u - r * nF;
+    int f, r;  // slab and token range
+    xcd_item((int)blockIdx.x, nF, R, a.n > a.rows, f, r);
     const int b0 = (int)((long)r * nTB / R), b1 = (int)((long)(r + 1) * nTB / R);
     if (b0 >= b1) return;
 
@@ -550,10 +546,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int rg = wave & 3, kh = wave >> 2;
-    const int G = gridDim.x, bid = blockIdx.x;
-    const int xcd = bid & 7, local = bid >> 3, q8 = G >> 3, r8 = G & 7;
-    const int u = xcd * q8 + (xcd < r8 ? xcd : r8) + local;
-    const int r = u / nF, f = u - r * nF;
+    int f, r;
+    xcd_item((int)blockIdx.x, nF, R, a.n > a.rows, f, r);
     const int b0 = (int)((long)r * nTB / R), b1 = (int)((long)(r + 1) * nTB / R);
     if (b0 >= b1) return;
 

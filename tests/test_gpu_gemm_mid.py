@@ -100,3 +100,18 @@ def test_row_major_equals_packed(rows, n, k, epi):
     torch.cuda.synchronize()
     assert torch.equal(out, again)
     assert np.isfinite(out.float().cpu().numpy()).all()
+
+
+def test_wide_output_stride():
+    """Output rows 2^26 elements apart: 16 of them are past a 32-bit byte offset, so the kernels that address them so
+    leave the call to the others.  Tolerance: 768 sums of bf16 products and half a bf16 step, as above."""
+    rows, n, k = 353, 2304, 768
+    x, w, _, want, size = _operands(rows, n, k, abi.EPI_STORE_BF16, 5, k)
+    out = torch.empty(rows, 1 << 26, device="cuda", dtype=BF16)  # 44 GiB, of which the first 2304 columns are touched
+    hip.op_gemm_splitk(abi.EPI_STORE_BF16, x, w, out, torch.empty(6 << 20, device="cuda"))
+    torch.cuda.synchronize()
+    got = out[:, :n].double()
+    del out
+    torch.cuda.empty_cache()
+    tol = 768 * 2.0 ** -24 * size + 2.0 ** -8 * want.abs() + 1e-6
+    assert bool(((got - want).abs() <= tol).all()), ((got - want).abs() - tol).max().item()
