@@ -81,15 +81,17 @@ __device__ inline void xcd_item(int b, int nF, int nR, bool slab_order, int& f, 
     r = slab_order ? lo : hi;
 }
 
-// v plus the same value of another lane, lanes paired as in a butterfly over 1, 2,
-// 4, 8 (within 16 lanes, by DPP: the mirrored orders pair the same partial sums),
-// 16 and 32: six VALU steps, where a shuffle through LDS took over 100 cycles each
-// (one request of 161 tokens, 43 LayerNorms in GEMM prologues: 734 -> 704 us).
+// v plus the same value of lane l ^ STEP, for a butterfly that takes its steps from
+// 32 down to 1, the order of sums that the wavefronts of this library have always
+// had: half-wave and 16-lane swaps, then DPP within 16 lanes (a rotation by 8, by 4
+// of values that repeat every 8, and quad permutations).  Six VALU steps, where a
+// shuffle through LDS took over 100 cycles each (one request of 161 tokens, 43
+// LayerNorms in GEMM prologues: 734 -> 704 us).
 template <int STEP>
 __device__ inline float lane_pair_sum(float v) {
     const int i = __builtin_bit_cast(int, v);
     if constexpr (STEP < 16) {
-        constexpr int ctrl = STEP == 1 ? 0xB1 : STEP == 2 ? 0x4E : STEP == 4 ? 0x141 : 0x140;
+        constexpr int ctrl = STEP == 1 ? 0xB1 : STEP == 2 ? 0x4E : STEP == 4 ? 0x124 : 0x128;
         return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, i, ctrl, 0xf, 0xf, true));
     } else if constexpr (STEP == 16) {
         const u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(i, i, false, false));
@@ -106,17 +108,17 @@ __device__ inline float lane_pair_sum(float v) {
 template <int N>
 __device__ inline void wave_sum_n(float (&v)[N]) {
 #pragma unroll
-    for (int r = 0; r < N; ++r) v[r] = lane_pair_sum<1>(v[r]);
-#pragma unroll
-    for (int r = 0; r < N; ++r) v[r] = lane_pair_sum<2>(v[r]);
-#pragma unroll
-    for (int r = 0; r < N; ++r) v[r] = lane_pair_sum<4>(v[r]);
-#pragma unroll
-    for (int r = 0; r < N; ++r) v[r] = lane_pair_sum<8>(v[r]);
+    for (int r = 0; r < N; ++r) v[r] = lane_pair_sum<32>(v[r]);
 #pragma unroll
     for (int r = 0; r < N; ++r) v[r] = lane_pair_sum<16>(v[r]);
 #pragma unroll
-    for (int r = 0; r < N; ++r) v[r] = lane_pair_sum<32>(v[r]);
+    for (int r = 0; r < N; ++r) v[r] = lane_pair_sum<8>(v[r]);
+#pragma unroll
+    for (int r = 0; r < N; ++r) v[r] = lane_pair_sum<4>(v[r]);
+#pragma unroll
+    for (int r = 0; r < N; ++r) v[r] = lane_pair_sum<2>(v[r]);
+#pragma unroll
+    for (int r = 0; r < N; ++r) v[r] = lane_pair_sum<1>(v[r]);
 }
 
 __device__ inline float wave_sum(float v) {

@@ -519,6 +519,26 @@ def test_final_norm_and_scorer():
     assert np.abs(host(s) - expect).max() < 1e-4
 
 
+@pytest.mark.parametrize("hidden", [64, 384, 768])
+def test_wave_sum_order(hidden):
+    """A wavefront's sum adds lanes l and l ^ 32, then ^ 16, 8, 4, 2 and 1, so a row's FP32 bits are those of a
+    butterfly in that order.  One element per lane is set; rows 0 .. 63 of the scorer give each lane's term by itself,
+    the last row their sum, bit for bit."""
+    r = rng(64)
+    vec = next(v for v in (4, 2, 1) if hidden // 64 % v == 0)
+    w2 = np.zeros(hidden, dtype=np.float32)
+    w2[np.arange(64) * vec] = r.standard_normal(64) * 2.0 ** r.integers(-12, 12, 64)
+    z = np.zeros((65, hidden), dtype=np.float32)
+    z[np.arange(64), np.arange(64) * vec] = z[64, np.arange(64) * vec] = 2.0
+    out = torch.zeros(65, device="cuda")
+    hip.op_scorer(dev(z), dev(w2), 0.0, out)
+    got = host(out).astype(np.float32)
+    s = got[:64].copy()
+    for step in (32, 16, 8, 4, 2, 1):
+        s = s + s[np.arange(64) ^ step]
+    assert np.all(s == s[0]) and got[64] == s[0], (got[64], s[0])
+
+
 def _attn_ref64(q, k, v, seqs, heads, window, scale=0.125):
     """f64 softmax(scale·QKᵀ + mask)·V per (sequence, head); seqs = (q_row, nq, kv_row, len, q_pos)."""
     out = np.zeros((q.shape[0], heads * 64))
