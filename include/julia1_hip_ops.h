@@ -192,8 +192,9 @@ typedef struct jh_attn_tile {
  * are dispatched in list order with heads varying fastest, so listing the
  * costliest tiles first (as the backend does) balances the CUs.  Few work
  * items (at most one for every two CUs, or two per CU over long rows) have
- * their keys split over two or four groups of waves, which adds a query's
- * partial sums in another order.
+ * their keys split over two or four groups of waves where kv_len is 513 or
+ * more, which adds such a query's partial sums in another order; rows of up to
+ * 512 keys get the same bits in any launch.
  * Replaces attention_rope/attention_plain (src/cuda/kernels.cu:274-391); RoPE
  * is applied by the producing GEMM's ROPE epilogue instead of on every load.
  */

@@ -116,7 +116,7 @@ __device__ __forceinline__ void attend(const AttnArgs& a, const AttnTile& tile, 
     int kbeg = 0, kend = tile.kv_len;
     if (a.window >= 0) {
         kbeg = max(0, tile.q_pos - a.window);
-        // (the same tiles, in the same groups, for the sub-items of any size)
+        // (tiles of the row's own grid, whatever query the item starts with)
         if (KS > 1) kbeg &= ~(KT - 1);
         kend = min(tile.kv_len, tile.q_pos + tile.nq + a.window);
     }
@@ -393,12 +393,16 @@ __device__ __forceinline__ void attend(const AttnArgs& a, const AttnTile& tile, 
     }
 }
 
-// 128-query items, KS > 1: those whose keys are too few for the split to pay (where
-// the caller does not say so in a.longest, the launch knows only their number) run as with KS = 1, on the first four waves.  Measured (us,
-// hidden 384, one row of 500 / 900 / 1500 / 3928 keys): KS 1 10.0 / 15.1 / 22.0
-// / 50.4, KS 4 10.9 / 14.3 / 18.6 / 39.0; KS 2 at two items per CU: 8 rows of
-// 900 keys 23.6 -> 23.9, 4 of 1500 31.4 -> 30.3, one of 8192 138 -> 129.
-constexpr int kSplitKeys4 = 832, kSplitKeys2 = 1152;
+// KS > 1: rows of too few keys run as with KS = 1, 128 queries on a workgroup's
+// first four waves, whatever their neighbours in the launch.  128-query items: where
+// the split does not pay.  Measured (us, hidden 384, one row of 500 / 900 / 1500 /
+// 3928 keys): KS 1 10.0 / 15.1 / 22.0 / 50.4, KS 4 10.9 / 14.3 / 18.6 / 39.0; KS 2
+// at two items per CU: 8 rows of 900 keys 23.6 -> 23.9, 4 of 1500 31.4 -> 30.3.
+// Items of 32 or 64 queries: from kSplitRow keys on.  Below, they gain 2 us at 500 keys
+// (9.9 -> 8.0), 0.3 at 161 (6.5 -> 6.2, which the host's call hides) and 1.5 to 3.5% of a
+// request, but would make the sums of a short row, which most rows are, depend on
+// what else is in the launch.
+constexpr int kSplitKeys4 = 832, kSplitKeys2 = 1152, kSplitRow = 513;
 
 // SUB workgroups share a tile of the list, each with 32 NW / KS of its queries.
 template <int NW, bool WIN, int KS = 1, int SUB = 1>
@@ -411,15 +415,16 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(KS == 4
     const int head = (int)(blockIdx.x % (unsigned)a.heads);
     const int item = (int)(blockIdx.x / (unsigned)a.heads);
     AttnTile tile = a.tiles[item / SUB];
+    const bool whole = KS > 1 && tile.kv_len < (SUBQ < 128 ? kSplitRow : KS == 4 ? kSplitKeys4 : kSplitKeys2);
     if constexpr (SUB > 1) {
         const int off = item % SUB * SUBQ;
-        if (off >= tile.nq) return;
+        if (off >= tile.nq || (whole && off % 128)) return;
         tile.q_row += off;
         tile.q_pos += off;
-        tile.nq = min(tile.nq - off, SUBQ);
+        tile.nq = min(tile.nq - off, whole ? 128 : SUBQ);
     }
-    if constexpr (KS > 1 && SUBQ == 128) {
-        if (tile.kv_len < (KS == 4 ? kSplitKeys4 : kSplitKeys2)) {
+    if constexpr (KS > 1) {
+        if (whole) {
             if (threadIdx.x >= 256) return;
             attend<4, WIN, 1>(a, tile, head, *(bf16_t(*)[2][2][KT * 64])smem);
             return;
@@ -453,15 +458,16 @@ void launch_items(const AttnArgs& a, hipStream_t s) {
     const bool win = a.window >= 0;
     // Few items leave SIMDs with one or two waves, or none.  The keys of each are
     // then split four (two) ways, and where the items are few for the CUs its
-    // queries over two or four workgroups too.  Not for rows of one key tile; the
+    // queries over two or four workgroups too.  Only for rows of kSplitRow keys or more; the
     // unsplit queries only over long rows (see kSplitKeys4), and not on window
     // layers, whose items have at most four or five key tiles.  Measured (us, one
     // row, hidden 384, full attention, 128-query items / four ways / and 64-query
-    // workgroups): 500 keys 9.9 / 10.9 / 8.0, 933 15.1 / 14.4 / 10.6, 1500 22.0 / 18.7
-    // / 13.8, 2500 34.4 / 26.7 / 20.4; a whole request, 128-query items / 64 / 32: 161
-    // tokens 671 / 666 / 659, 300 763 / 741 / 736, 1200 1177 / 1121 / 1125; 30 tokens
-    // 603 / 614 / 622.
-    const bool split = a.key_split && (!a.longest || a.longest > KT);
+    // workgroups): 933 keys 15.1 / 14.4 / 10.6, 1500 22.0 / 18.7 / 13.8, 2500 34.4 / 26.7 /
+    // 20.4; a whole request of 1200 tokens, 128-query items / 64 / 32: 1177 / 1121 / 1125.
+    // Where the caller does not say how long the rows are, a list too short to cover
+    // one of kSplitRow queries runs unsplit: it would be run so anyway, and the larger
+    // kernel's LDS and empty workgroups cost 0.1 us of 6.7 at 161 keys.
+    const bool split = a.key_split && (a.longest ? a.longest >= kSplitRow : (long)a.ntiles * TQ >= kSplitRow);
     if (split && 8 * items <= cus) {
         if (win) JH_LAUNCH((attention_kernel<4, true, 4, TQ / 32>), grid(TQ / 32), dim3(256), 0, s, a);
         else JH_LAUNCH((attention_kernel<4, false, 4, TQ / 32>), grid(TQ / 32), dim3(256), 0, s, a);

@@ -527,10 +527,7 @@ struct jh_model {
                    long ldo, const AttnTile* tiles, size_t n, int nheads, int window, double pairs, double qrows,
                    int waves = 4) {
         AttnArgs a{q, ldq, k, v, ldkv, out, ldo, tiles, (int)n, nheads, window, 0.125f * 1.4426950408889634f, waves};
-        // Up to 512 tokens the splits gain 1.5 to 3.5% of a request, but a row alone
-        // would then differ in every attention layer from the same row in a larger
-        // batch: logits moved by up to 2.1e-3, past the 2e-3 that split-K keeps to.
-        a.key_split = use_splitk && longest > 512;
+        a.key_split = use_splitk;
         a.longest = (int)longest;
         const double hd = 64.0 * nheads;
         timed(cls, 4.0 * hd * pairs, qrows * hd * 2 * 2 + (double)T * hd * 2 * 2, [&] { launch_attention(a, stream); });

@@ -737,12 +737,12 @@ def test_attention_full_length_8192(window):
 @pytest.mark.parametrize("rate", [0.0, 0.4])
 @pytest.mark.parametrize("window", [-1, 64, 8])
 @pytest.mark.parametrize("heads,lens,wide", [
-    (2, [30, 161, 64, 65, 129], False),    # at most 32 items: 32-query workgroups, keys split four ways
+    (2, [513, 700, 30], False),            # at most 32 items: 32-query workgroups, keys split four ways from 513 keys on
     (2, [831, 832, 300, 960, 1], False),   # at most 128: 64-query workgroups
     (6, [831, 832, 833, 1], False),        # at most one 128-query item per CU: split from 832 keys on
     (12, [1151, 1152, 1153, 130], False),  # up to two per CU: two ways from 1152 on
     (12, [1407, 1300], True),              # 256-query tiles run as two 128-query workgroups each
-    (2, [300, 257], True),                 # ... and as eight of 32 queries
+    (2, [900, 257], True),                 # ... and as eight of 32 queries
 ])
 def test_attention_key_split(heads, lens, wide, window, rate):
     """Few work items: groups of waves take every second or fourth key tile and merge their running maxima, sums and
@@ -770,6 +770,31 @@ def test_attention_key_split(heads, lens, wide, window, rate):
                      dev(np.array(_tiles(lens, 256 if wide else 128), dtype=np.int32)), heads, window, wide=wide)
     assert np.abs(qkv[:, 2 * h:]).max() < 5.5
     assert np.abs(host(out) - expect).max() < 2.0 ** -8 * 5.5, np.abs(host(out) - expect).max()
+
+
+@pytest.mark.parametrize("window", [-1, 64, 8])
+@pytest.mark.parametrize("wide", [False, True])
+def test_attention_short_rows_in_any_launch(wide, window):
+    """Rows of up to 512 keys have one order of sums: alone (where few items would have their keys split), with a long
+    row beside them, and among enough rows that nothing is split, they get the same bits."""
+    heads, lens = 2, [512, 300, 65, 1]
+    h, t = heads * 64, sum(lens)
+    g = torch.Generator("cuda").manual_seed(513)
+    fill = 66 * 512
+    qkv = torch.randn(t + fill, 3 * h, device="cuda", generator=g).to(BF16)
+
+    def rows(ls, qt, wide):
+        n = sum(ls)
+        out = torch.zeros(n, h, dtype=BF16, device="cuda")
+        hip.op_attention(qkv, 3 * h, qkv[:, h:], qkv[:, 2 * h:], 3 * h, out, h,
+                         dev(np.array(_tiles(ls, qt), dtype=np.int32)), heads, window, wide=wide)
+        return out[:t]
+
+    qt = 256 if wide else 128
+    want = rows(lens + [512] * 66, 128, False)
+    assert torch.equal(rows(lens, qt, wide), want)
+    assert torch.equal(rows(lens + [900], qt, wide), want)
+    assert torch.equal(rows(lens[2:] + lens[:2], qt, wide), rows(lens[2:] + lens[:2] + [512] * 66, 128, False))
 
 
 def test_attention_marker_queries():
