@@ -207,14 +207,24 @@ int jh_op_attention(const void* q, size_t ldq, const void* k, const void* v, siz
  * eight waves per (tile, head), each staged K/V tile shared by twice the
  * queries, or two 128-query workgroups per tile where those leave fewer CUs
  * idle (and on window layers).  The backend uses it for the global layers of
- * sequences of 4096 tokens or more.  Same arithmetic per query as
- * jh_op_attention for the same number of workgroups.  No separate
- * counterpart in the reference (part of attention_rope/attention_plain,
- * src/cuda/kernels.cu:274-391).
+ * sequences of 4096 tokens or more.  Keys are split over few items as in
+ * jh_op_attention.  No separate counterpart in the reference (part of
+ * attention_rope/attention_plain, src/cuda/kernels.cu:274-391).
  */
 int jh_op_attention_wide(const void* q, size_t ldq, const void* k, const void* v, size_t ldkv,
                          void* out, size_t ldo, const jh_attn_tile* tiles, size_t ntiles,
                          size_t heads, int window, float scale, void* stream);
+
+/*
+ * jh_op_attention (wide = 0) or jh_op_attention_wide (wide != 0) with no key
+ * split: every query's keys are added by one wave in one order, so a row gets the
+ * same bits whatever else is in the launch, and from both item sizes where they
+ * cut the row at multiples of 128 and 256.  What the backend runs after
+ * jh_set_splitk(model, 0).  No reference counterpart.
+ */
+int jh_op_attention_unsplit(const void* q, size_t ldq, const void* k, const void* v, size_t ldkv,
+                            void* out, size_t ldo, const jh_attn_tile* tiles, size_t ntiles,
+                            size_t heads, int window, float scale, int wide, void* stream);
 
 #ifdef __cplusplus
 }

@@ -13,6 +13,18 @@ inline int as_int(size_t v, const char* what) {
     if (v > (size_t)0x7fffffff) throw jh_error(JH_ERR_INVALID, std::string(what) + " too large");
     return (int)v;
 }
+
+int op_attention(const void* q, size_t ldq, const void* k, const void* v, size_t ldkv, void* out, size_t ldo,
+                 const jh_attn_tile* tiles, size_t ntiles, size_t heads, int window, float scale, int waves,
+                 bool key_split, void* stream) {
+    return jh_guarded([&] {
+        static_assert(sizeof(jh_attn_tile) == sizeof(AttnTile), "tile layout");
+        AttnArgs a{(const bf16_t*)q, (long)ldq, (const bf16_t*)k, (const bf16_t*)v, (long)ldkv, (bf16_t*)out,
+                   (long)ldo, (const AttnTile*)tiles, as_int(ntiles, "ntiles"), as_int(heads, "heads"), window,
+                   scale * 1.4426950408889634f, waves, key_split};
+        launch_attention(a, (hipStream_t)stream);
+    });
+}
 }  // namespace
 
 extern "C" {
@@ -133,24 +145,19 @@ int jh_op_scorer(const float* z, size_t rows, size_t hidden, const float* w2, fl
 
 int jh_op_attention(const void* q, size_t ldq, const void* k, const void* v, size_t ldkv, void* out, size_t ldo,
                     const jh_attn_tile* tiles, size_t ntiles, size_t heads, int window, float scale, void* stream) {
-    return jh_guarded([&] {
-        static_assert(sizeof(jh_attn_tile) == sizeof(AttnTile), "tile layout");
-        AttnArgs a{(const bf16_t*)q, (long)ldq, (const bf16_t*)k, (const bf16_t*)v, (long)ldkv, (bf16_t*)out,
-                   (long)ldo, (const AttnTile*)tiles, as_int(ntiles, "ntiles"), as_int(heads, "heads"), window,
-                   scale * 1.4426950408889634f};
-        launch_attention(a, (hipStream_t)stream);
-    });
+    return op_attention(q, ldq, k, v, ldkv, out, ldo, tiles, ntiles, heads, window, scale, 4, true, stream);
 }
 
 int jh_op_attention_wide(const void* q, size_t ldq, const void* k, const void* v, size_t ldkv, void* out, size_t ldo,
                          const jh_attn_tile* tiles, size_t ntiles, size_t heads, int window, float scale,
                          void* stream) {
-    return jh_guarded([&] {
-        AttnArgs a{(const bf16_t*)q, (long)ldq, (const bf16_t*)k, (const bf16_t*)v, (long)ldkv, (bf16_t*)out,
-                   (long)ldo, (const AttnTile*)tiles, as_int(ntiles, "ntiles"), as_int(heads, "heads"), window,
-                   scale * 1.4426950408889634f, 8};
-        launch_attention(a, (hipStream_t)stream);
-    });
+    return op_attention(q, ldq, k, v, ldkv, out, ldo, tiles, ntiles, heads, window, scale, 8, true, stream);
+}
+
+int jh_op_attention_unsplit(const void* q, size_t ldq, const void* k, const void* v, size_t ldkv, void* out,
+                            size_t ldo, const jh_attn_tile* tiles, size_t ntiles, size_t heads, int window,
+                            float scale, int wide, void* stream) {
+    return op_attention(q, ldq, k, v, ldkv, out, ldo, tiles, ntiles, heads, window, scale, wide ? 8 : 4, false, stream);
 }
 
 }  // extern "C"

@@ -597,12 +597,16 @@ def test_attention_varlen(window, qt):
 
 
 @pytest.mark.parametrize("window", [-1, 64])
-def test_attention_wide_items(window):
+@pytest.mark.parametrize("heads,key_split", [
+    (2, False),  # 36 tiles of 256 queries: two 128-query workgroups each
+    (8, False),  # 144: full attention on the eight-wave kernel, one per tile
+    (2, True),   # rows of 700 and 1300 keys split four ways, both item sizes in 64-query workgroups
+])
+def test_attention_wide_items(heads, key_split, window):
     """jh_op_attention_wide (eight waves, up to 256 queries per work item; the backend's global layers of long
     sequences) on ragged lengths: each query's keys are visited in the same 64-key tiles as with 128-query items,
     so the output equals jh_op_attention's bit for bit, and both are within 2e-2 of the f64 reference."""
     r = rng(31)
-    heads = 2
     h = heads * 64
     lens = [1, 100, 129, 255, 256, 257, 511, 700, 1300]
     t = sum(lens)
@@ -617,21 +621,29 @@ def test_attention_wide_items(window):
     for qt, wide in ((128, False), (256, True)):
         out = torch.zeros(t, h, dtype=BF16, device="cuda")
         hip.op_attention(dq, 3 * h, dq[:, h:], dq[:, 2 * h:], 3 * h, out, h,
-                         dev(np.array(_tiles(lens, qt), dtype=np.int32)), heads, window, wide=wide)
+                         dev(np.array(_tiles(lens, qt), dtype=np.int32)), heads, window, wide=wide,
+                         key_split=key_split)
         outs.append(host(out))
     assert np.array_equal(outs[0], outs[1])
     assert np.abs(outs[1] - expect).max() < 2e-2, np.abs(outs[1] - expect).max()
 
 
 @pytest.mark.parametrize("window", [-1, 64])
-def test_attention_rising_scores(window):
+@pytest.mark.parametrize("heads,lens,key_split", [
+    (2, [300, 257, 300, 190, 300], False),
+    (2, [300, 257, 300, 190, 300], True),        # rows under 513 keys: as without the split
+    (2, [833, 900], True),                       # four ways, 32-query workgroups
+    (2, [900, 1025, 833, 1100, 1300], True),     # four ways, 64-query workgroups
+    (5, [900, 1025, 833, 1100, 1300], True),     # four ways, 128-query items (full attention)
+    (12, [1200, 1300, 1152], True),              # two ways (full attention)
+])
+def test_attention_rising_scores(heads, lens, key_split, window):
     """Scores that climb along each sequence at several rates (about 2 to 40 log2 units per 64-key tile), so the
     running max must move again and again after the first tile: every rescale case of the online softmax (a rise
-    within the lazy threshold, just past it, far past it, to where exp2 would overflow without one) against f64."""
+    within the lazy threshold, just past it, far past it, to where exp2 would overflow without one) against f64.
+    The split rows have at least three tiles per group of waves, so each group rescales again and again too."""
     r = rng(11)
-    heads = 2
     h = heads * 64
-    lens = [300, 257, 300, 190, 300]
     rates = [0.15, 0.5, 0.8, 1.3, 3.0]  # beta rise per 64 keys
     t = sum(lens)
     q = np.abs(r.standard_normal((t, h))) + 0.5
@@ -654,31 +666,44 @@ def test_attention_rising_scores(window):
     dq = dev(qkv, BF16)
     out = torch.zeros(t, h, dtype=BF16, device="cuda")
     hip.op_attention(dq, 3 * h, dq[:, h:], dq[:, 2 * h:], 3 * h, out, h, dev(np.array(tiles, dtype=np.int32)), heads,
-                     window)
+                     window, key_split=key_split)
     got = host(out)
     assert np.isfinite(got).all()
     assert np.abs(got - expect).max() < 2e-2, np.abs(got - expect).max()
 
 
-@pytest.mark.parametrize("window", [-1, 512])
-def test_attention_scores_far_above_running_max(window):
+@pytest.mark.parametrize("window", [-1, 2048])
+@pytest.mark.parametrize("heads,groups,group,pad", [
+    (2, 1, 0, 0),    # keys not split: tiles 0 .. 3 of each row
+    (2, 4, 0, 0),    # four ways, 32-query workgroups: the first group's tiles
+    (2, 4, 3, 0),    # ... the last group's
+    (8, 4, 1, 0),    # four ways, 64-query workgroups
+    (16, 4, 2, 0),   # four ways, 128-query items (full attention)
+    (16, 2, 1, 12),  # two ways (full attention, 1152 keys or more)
+])
+def test_attention_scores_far_above_running_max(heads, groups, group, pad, window):
     """Single keys whose scores sit 12 to 15 log2 units above the running max (scores ~0 before them).  The fast
     path keeps a tile without computing its max while each lane's 32 values of p sum to at most 2^16, so it
     carries one p of up to 2^15 (keys 70 and 100 share a lane: 2^12 + 2^13.5); two keys at 15.5 units in one
     lane's 32 (keys 192, 193) exceed the bound and send that tile to the slow path, which moves the max; a spike in a
-    sequence's last, partial tile (key 199 of 200) is masked on the slow path.  Against f64 softmax.  (Window 512
-    covers both sequences, so no tile is a window edge and the fast path runs as for global attention.)"""
+    sequence's last, partial tile (key 199 of 200) is masked on the slow path.  Against f64 softmax.  (Window 2048
+    covers both sequences, so no tile is a window edge and the fast path runs as for global attention.)  Where keys
+    are split over groups of waves, those four tiles are consecutive ones of one group, `pad` tiles into the row."""
     r = rng(12)
-    heads = 2
     h = heads * 64
-    lens = [256, 200]
+
+    def key(i):  # key i of the unsplit rows
+        return (pad + group + groups * (i // 64)) * 64 + i % 64
+
+    lens = [key(255) + 1, key(199) + 1]
     t = sum(lens)
     c = 0.125 * math.log2(math.e)
     u = np.abs(r.standard_normal(h)) + 0.5
-    q = u[None, :] + 0.05 * r.standard_normal((t, h))
+    # (a spike errs by 15 (noise / |u|) times a normal variate, 0.08 log2 units at 0.05: more rows and heads draw further out)
+    q = u[None, :] + (0.05 if groups == 1 else 0.03) * r.standard_normal((t, h))
     k = 0.05 * r.standard_normal((t, h))
-    spikes = [(70, 12.0), (100, 13.5), (150, 15.0), (192, 15.5), (193, 15.5),
-              (256 + 64, 14.0), (256 + 130, 12.5), (256 + 199, 15.0)]
+    spikes = [(key(70), 12.0), (key(100), 13.5), (key(150), 15.0), (key(192), 15.5), (key(193), 15.5),
+              (lens[0] + key(64), 14.0), (lens[0] + key(130), 12.5), (lens[0] + key(199), 15.0)]
     for row, d in spikes:
         for hh in range(heads):
             uh = u[hh * 64:(hh + 1) * 64]
@@ -702,7 +727,7 @@ def test_attention_scores_far_above_running_max(window):
     dq = dev(qkv, BF16)
     out = torch.zeros(t, h, dtype=BF16, device="cuda")
     hip.op_attention(dq, 3 * h, dq[:, h:], dq[:, 2 * h:], 3 * h, out, h, dev(np.array(tiles, dtype=np.int32)), heads,
-                     window)
+                     window, key_split=groups > 1)
     got = host(out)
     assert np.isfinite(got).all()
     assert np.abs(got - expect).max() < 2e-2, np.abs(got - expect).max()
