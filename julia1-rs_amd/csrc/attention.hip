@@ -476,8 +476,9 @@ void launch_items(const AttnArgs& a, hipStream_t s) {
         else JH_LAUNCH((attention_kernel<8, false, 4, TQ / 64>), grid(TQ / 64), dim3(512), 0, s, a);
     } else if (split && !win && items <= cus && (!a.longest || a.longest >= kSplitKeys4)) {
         JH_LAUNCH((attention_kernel<16, false, 4, TQ / 128>), grid(TQ / 128), dim3(1024), 0, s, a);
-    } else if (split && !win && items > cus && items <= 2 * cus && (!a.longest || a.longest >= kSplitKeys2)) {
-        JH_LAUNCH((attention_kernel<8, false, 2, TQ / 128>), grid(TQ / 128), dim3(512), 0, s, a);
+    } else if (TQ == 128 && split && !win && items > cus && items <= 2 * cus && (!a.longest || a.longest >= kSplitKeys2)) {
+        // (256-query tiles of this number run whole: see wide_cost)
+        JH_LAUNCH((attention_kernel<8, false, 2>), grid(1), dim3(512), 0, s, a);
     } else if (win) {
         JH_LAUNCH((attention_kernel<4, true, 1, TQ / 128>), grid(TQ / 128), dim3(256), 0, s, a);
     } else {

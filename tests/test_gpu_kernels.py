@@ -766,7 +766,9 @@ def test_attention_full_length_8192(window):
     (2, [831, 832, 300, 960, 1], False),   # at most 128: 64-query workgroups
     (6, [831, 832, 833, 1], False),        # at most one 128-query item per CU: split from 832 keys on
     (12, [1151, 1152, 1153, 130], False),  # up to two per CU: two ways from 1152 on
-    (12, [1407, 1300], True),              # 256-query tiles run as two 128-query workgroups each
+    (12, [1407, 1300], True),              # 144 tiles of 256 queries: the eight-wave kernel, unsplit (full attention)
+    (6, [1407, 1300], True),               # 72: as two 128-query workgroups each, split four ways (full attention)
+    (32, [1407, 1300], True),              # 384: as two 128-query workgroups each, unsplit
     (2, [900, 257], True),                 # ... and as eight of 32 queries
 ])
 def test_attention_key_split(heads, lens, wide, window, rate):
