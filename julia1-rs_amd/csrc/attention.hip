@@ -496,10 +496,13 @@ void launch_attention(const AttnArgs& a, hipStream_t s) {
     if (a.ldq % 8 || a.ldkv % 8 || a.ldo % 4 || a.ldq < a.heads * 64 || a.ldo < a.heads * 64 ||
         ((uintptr_t)a.q & 15) || ((uintptr_t)a.k & 15) || ((uintptr_t)a.v & 15) || ((uintptr_t)a.out & 7))
         throw jh_error(1, "attention: operands must be 16-byte aligned with row strides % 8 == 0");
-    if ((long)a.ntiles * a.heads > 0x0fffffffL) throw jh_error(1, "attention: grid too large");
-    const long cus = gemm_resident_tiles() / 2, items = (long)a.ntiles * a.heads;
+    // Workgroups: one per item, two for a tile run as halves (more only where items are few).
+    const long items = (long)a.ntiles * a.heads, most = 0x7fffffffL;
+    if (items > most || (a.waves == 8 && a.window >= 0 && 2 * items > most))
+        throw jh_error(1, "attention: grid too large");
+    const long cus = gemm_resident_tiles() / 2;
     if (a.waves == 4) launch_items<128>(a, s);
-    else if (a.window >= 0 || halves_cost(items, cus) < wide_cost(items, cus)) launch_items<256>(a, s);
+    else if (a.window >= 0 || (2 * items <= most && halves_cost(items, cus) < wide_cost(items, cus))) launch_items<256>(a, s);
     else JH_LAUNCH((attention_kernel<8, false>), dim3((unsigned)items), dim3(512), 0, s, a);
     HIP_CHECK(hipGetLastError());
 }

@@ -63,6 +63,25 @@ def test_create_without_device_reports_error_not_crash():
     assert e.value.code == 2
 
 
+@pytest.mark.skipif(os.path.exists("/dev/kfd"), reason="calls that pass the checks would be launched")
+@pytest.mark.parametrize("entry,window,ntiles,heads,refused", [
+    ("jh_op_attention", -1, 0x10000000, 1, False),
+    ("jh_op_attention", 64, 0x7fffffff, 1, False),
+    ("jh_op_attention", -1, 0x40000000, 2, True),
+    ("jh_op_attention_wide", -1, 0x7fffffff, 1, False),
+    ("jh_op_attention_wide", 64, 0x10000000, 3, False),
+    ("jh_op_attention_wide", 64, 0x40000000, 1, True),   # two workgroups per tile
+])
+def test_attention_item_limit(entry, window, ntiles, heads, refused):
+    """Attention refuses more workgroups than a grid holds, and no fewer: without a GPU, a call that passes the checks
+    fails at the device instead."""
+    L, p = hip.lib(), 1 << 20
+    rc = getattr(L, entry)(p, 64 * heads, p, p, 64 * heads, p, 64 * heads, p, ntiles, heads, window, 0.125, None)
+    message = L.jh_last_error().decode()
+    assert rc == (abi.JH_ERR_INVALID if refused else abi.JH_ERR_DEVICE), (rc, message)
+    assert ("grid too large" in message) == refused, message
+
+
 def test_create_rejects_bad_config_before_touching_device():
     cfg = synth.model_config("tiny")
     ws = abi.WeightSet(cfg, synth.make_weights(cfg, 0))
