@@ -27,8 +27,9 @@
 // chunks XOR-swizzled by (row >> 1) & 7 as in gemm.hip (conflict-free B-fragment
 // reads).  RoPE cos/sin rows of the block's tokens are gathered into LDS by DMA.
 //
-// Schedule.  Workgroups are (token range, feature slab) pairs, dealt so that
-// the slabs sharing a token range sit on one XCD (X read once per L2).  Per
+// Schedule.  Workgroups are (token range, feature slab) pairs, dealt to the XCDs
+// (xcd_item) so that the slabs sharing a token range sit on one, X then being read
+// once per L2, or, where N > tokens, the ranges sharing a slab, and W is.  Per
 // 16-token block: one barrier; then every wave runs the block's 48 MFMAs and,
 // between them, issues its share of the next block's X DMA (into the other of
 // two X slots) and runs the previous block's epilogue from its second set of
