@@ -1228,7 +1228,8 @@ int resident_tiles() {
 }
 
 // Tile width (64 or 32 features) of the one-launch small-batch kernel for
-// `a`, or 0 when launch_gemm does not use it.  It replaces split-K where
+// `a`, or 0 when it does not take it (launch_cfg asks slab_waves and ws_takes
+// first).  It replaces split-K where
 // split-K would run automatically (workspace given, no forced split count)
 // and K fits its LDS; with the LayerNorm prologue it is the only kernel.
 // 32-feature tiles move fewer operand bytes per CU, so they are taken when
@@ -1498,7 +1499,8 @@ int gemm_splitk_count(int epi, const GemmArgs& a) {
 }
 
 bool gemm_uses_small(int epi, const GemmArgs& a) {
-    return validate_gemm(epi, a) && small_bf(epi, a) != 0;
+    // in launch_cfg's order
+    return validate_gemm(epi, a) && !slab_waves(a) && !(a.splits == 0 && ws_takes(epi, a)) && small_bf(epi, a) != 0;
 }
 
 void launch_gemm_partial(int epi, const GemmArgs& a, int splits, hipStream_t s) {

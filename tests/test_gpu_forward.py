@@ -291,6 +291,25 @@ def test_hidden_384_shape(shape):
         check_gates(s)
 
 
+@pytest.mark.parametrize("tokens,fused", [(1024, True), (1025, False), (1280, False)])
+def test_fused_small_layers_only_on_the_small_kernel(tokens, fused):
+    """The LayerNorms move into the small-batch GEMMs' prologues only where all four projections of a layer run as
+    small-batch launches.  At hidden 384 with a GEGLU width of 768, Wi goes to the slab-resident kernel from 1025
+    tokens on, so from there the layers keep their LayerNorm launches; scores match the oracle on both sides."""
+    shape = synth.SHAPES["julia1-384"]
+    cfg = abi.ModelConfig.from_values(shape["julia"], dict(shape["enc"], intermediate_size=768))
+    ws = abi.WeightSet(cfg, synth.make_weights(cfg, seed=6))
+    gpu, orc = hip.HipModel(ws), oracle.OracleModel(ws, threads=8)
+    b = synth.make_batch([tokens], [5], cfg.vocab, 23)
+    gpu.profile(True)
+    got = gpu.forward(b)
+    launches = {s["name"]: s["launches"] for s in gpu.profile_read()}
+    gpu.profile(False)
+    assert (launches.get("layer_norm", 0) == 0) == fused, launches
+    check_gates(parity(b, got, orc.forward(b)))
+    gpu.close()
+
+
 def test_base_config4_slice(base):
     """32 rows of the router-scale varlen batch against the oracle."""
     ws, gpu, orc = base
