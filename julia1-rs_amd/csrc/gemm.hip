@@ -1245,10 +1245,9 @@ int small_bf(int epi, const GemmArgs& a) {
     return a.k <= small_kmax<64>() ? 64 : 0;
 }
 
-// Row strides with which the slab-resident and weight-stationary kernels may stand
-// in for the small-batch and split-K ones: they address 16 rows of X and of the
-// output with 32-bit byte offsets (16 * 2^24 floats are 2^30 bytes), the others the
-// output with 64-bit addresses.
+// Row strides with which the slab-resident and weight-stationary kernels stand in
+// for the small-batch and split-K ones: those address the output with 64-bit
+// addresses, these must pass gemm_offsets_fit (16 * 2^24 floats are 2^30 bytes).
 bool narrow_strides(const GemmArgs& a) { return a.ldx <= 1L << 24 && a.ldo <= 1L << 24; }
 
 // Waves per workgroup of the slab-resident kernel (K = 384) for `a`, or 0 when
@@ -1264,8 +1263,8 @@ bool narrow_strides(const GemmArgs& a) { return a.ldx <= 1L << 24 && a.ldo <= 1L
 //     and a half rounds to the small-batch kernel's last size;
 //   twelve waves (384-row slabs), N = 1152: 9500 15.5 / 17.7, 16384 24.0 / 24.0,
 //     65536 96 / 66; N = 2304: 16384 38.9 / 37.1, 65536 167 / 124.
-int slab_waves(const GemmArgs& a) {
-    if (!a.partial || a.splits != 0 || !gemm_slab_supported(a) || !narrow_strides(a)) return 0;
+int slab_waves(int epi, const GemmArgs& a) {
+    if (!a.partial || a.splits != 0 || !gemm_slab_supported(epi, a) || !narrow_strides(a)) return 0;
     if (a.rows >= 16384 && a.n >= 1024 && a.n % 384 == 0) return 12;
     const long cus = resident_tiles() / 2, tiles = (long)((a.n + 127) / 128) * ((a.rows + 127) / 128);
     const long small = (long)(a.n / 64) * ((a.rows + SMALL_BT - 1) / SMALL_BT);
@@ -1404,7 +1403,7 @@ template <int EPI>
 void launch_cfg(const GemmArgs& a, hipStream_t s) {
     constexpr int BF = 128, BT = 128;
     const int blocks = ((a.n + BF - 1) / BF) * ((a.rows + BT - 1) / BT);
-    if (const int waves = slab_waves(a)) {
+    if (const int waves = slab_waves(EPI, a)) {
         launch_gemm_slab(EPI, a, waves, s);
         return;
     }
@@ -1429,7 +1428,7 @@ void launch_cfg(const GemmArgs& a, hipStream_t s) {
         HIP_CHECK(hipGetLastError());
         return;
     }
-    if (gemm_ws_supported(EPI, a)) {  // a forced split count that K does not allow
+    if (gemm_ws_supported(EPI, a)) {  // packed W that no rule above, nor a split of K, took
         launch_gemm_ws(EPI, a, s);
         return;
     }
@@ -1494,13 +1493,13 @@ int gemm_resident_tiles() { return resident_tiles(); }
 bool validate_gemm_args(int epi, const GemmArgs& a) { return validate_gemm(epi, a); }
 
 int gemm_splitk_count(int epi, const GemmArgs& a) {
-    if (!validate_gemm(epi, a) || slab_waves(a) || (a.splits == 0 && ws_takes(epi, a))) return 1;
+    if (!validate_gemm(epi, a) || slab_waves(epi, a) || (a.splits == 0 && ws_takes(epi, a))) return 1;
     return splitk_count(a, (long)((a.n + 127) / 128) * ((a.rows + 127) / 128));
 }
 
 bool gemm_uses_small(int epi, const GemmArgs& a) {
     // in launch_cfg's order
-    return validate_gemm(epi, a) && !slab_waves(a) && !(a.splits == 0 && ws_takes(epi, a)) && small_bf(epi, a) != 0;
+    return validate_gemm(epi, a) && !slab_waves(epi, a) && !(a.splits == 0 && ws_takes(epi, a)) && small_bf(epi, a) != 0;
 }
 
 void launch_gemm_partial(int epi, const GemmArgs& a, int splits, hipStream_t s) {

@@ -328,8 +328,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 4
 
 }  // namespace
 
-bool gemm_slab_supported(const GemmArgs& a) {
-    return a.k == SL_K && a.n % 128 == 0 && !a.gather && !a.xf && a.rows > 0 && a.w;
+bool gemm_slab_supported(int epi, const GemmArgs& a) {
+    return a.k == SL_K && a.n % 128 == 0 && !a.gather && !a.xf && a.rows > 0 && a.w && gemm_offsets_fit(epi, a);
 }
 
 namespace {
@@ -355,8 +355,9 @@ void launch_slab(int epi, const GemmArgs& a, int nF, int R, int nU, hipStream_t 
 }  // namespace
 
 void launch_gemm_slab(int epi, const GemmArgs& a, int waves, hipStream_t s) {
-    if (!gemm_slab_supported(a) || (waves != 4 && (waves != 12 || a.n % 384)))
-        throw jh_error(1, "gemm: the slab kernel needs K = 384 and N a multiple of its 128 or 384 rows");
+    if (!gemm_slab_supported(epi, a) || (waves != 4 && (waves != 12 || a.n % 384)))
+        throw jh_error(1, "gemm: the slab kernel needs K = 384 and N a multiple of its 128 or 384 rows, and rows of X "
+                          "and the output under 2^28 bytes");
     // Token ranges per slab: as many as give two workgroups of four waves, or one
     // of twelve, per CU; at least one unit each.
     const int nU = (a.rows + SL_UNIT - 1) / SL_UNIT, slots = gemm_resident_tiles() / (waves == 4 ? 1 : 2);

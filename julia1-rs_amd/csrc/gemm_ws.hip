@@ -765,7 +765,7 @@ int device_cus() {
 }  // namespace
 
 bool gemm_ws_shape(int epi, const GemmArgs& a) {
-    if (a.gather || a.xf || a.rows <= 0) return false;
+    if (a.gather || a.xf || a.rows <= 0 || !gemm_offsets_fit(epi, a)) return false;
     if (a.k == W2_K) return a.n % W2_ROWS == 0 && epi == JH_EPI_RESID_F32;
     return a.k == WS_K && a.n % WS_ROWS == 0 && epi >= JH_EPI_STORE_BF16 && epi <= JH_EPI_BIAS_F32;
 }
@@ -811,8 +811,8 @@ static void launch_ws(int epi, const GemmArgs& a, hipStream_t s) {
 
 void launch_gemm_ws(int epi, const GemmArgs& a, hipStream_t s) {
     if (!(a.w_ws ? gemm_ws_supported(epi, a) : gemm_ws_shape(epi, a) && a.w))
-        throw jh_error(1, "gemm: weight-stationary kernel needs packed W and K = 768 with N % 256 == 0, or K = 1152 "
-                          "with N % 128 == 0 and the residual epilogue");
+        throw jh_error(1, "gemm: weight-stationary kernel needs K = 768 with N % 256 == 0, or K = 1152 with N % 128 == 0 "
+                          "and the residual epilogue, and rows of X and the output under 2^28 bytes");
     if (a.w_ws) launch_ws<false>(epi, a, s);
     else launch_ws<true>(epi, a, s);
 }

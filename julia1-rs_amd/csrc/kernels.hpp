@@ -74,8 +74,16 @@ int gemm_splitk_count(int epilogue, const GemmArgs& a);
 // only kernel with the LayerNorm prologue); false for rows == 0.
 bool gemm_uses_small(int epilogue, const GemmArgs& a);
 void launch_gemm_partial(int epilogue, const GemmArgs& a, int splits, hipStream_t stream);
-// Weight-stationary kernel (gemm_ws.hip): K = 768, N % 256 == 0, a.w_ws set,
-// no gather or LayerNorm prologue.  gemm_ws_ranges is the number of token
+// Whether 16 rows of X and of the output lie within 32-bit byte offsets, with which
+// the weight-stationary and slab-resident kernels address them (past that an
+// offset wraps onto another row); rows of 2^26 floats or 2^27 bf16 do not.
+inline bool gemm_offsets_fit(int epilogue, const GemmArgs& a) {
+    const long esz = epilogue == 3 || epilogue == 6 ? 4 : 2;  // JH_EPI_RESID_F32, JH_EPI_BIAS_F32
+    return a.ldx <= 0xffffffffL / (16 * 2) && a.ldo <= 0xffffffffL / (16 * esz);
+}
+// Weight-stationary kernel (gemm_ws.hip): K = 768, N % 256 == 0, or K = 1152, N % 128
+// == 0 and the residual epilogue; a.w_ws set, strides as above, no gather or LayerNorm
+// prologue.  gemm_ws_ranges is the number of token
 // ranges each 256-row slab is split into (one workgroup per CU).
 bool gemm_ws_supported(int epilogue, const GemmArgs& a);
 // The same but for W: launch_gemm_ws reads a.w, row-major, where a.w_ws is null.
@@ -88,9 +96,9 @@ int gemm_ws_block_tokens();
 void launch_gemm_ws(int epilogue, const GemmArgs& a, hipStream_t stream);
 void pack_ws(const bf16_t* w, int n, int k, bf16_t* out);
 
-// Slab-resident kernel (gemm_slab.hip): K = 384, N % 128 == 0, no gather or
-// LayerNorm prologue; every epilogue.  `waves` per workgroup: 4, or 12 (N % 384 == 0).
-bool gemm_slab_supported(const GemmArgs& a);
+// Slab-resident kernel (gemm_slab.hip): K = 384, N % 128 == 0, strides as above, no
+// gather or LayerNorm prologue; every epilogue.  `waves` per workgroup: 4, or 12 (N % 384 == 0).
+bool gemm_slab_supported(int epilogue, const GemmArgs& a);
 void launch_gemm_slab(int epi, const GemmArgs& a, int waves, hipStream_t stream);
 // 256-thread workgroups with at most 80 KB of LDS that the current device
 // holds at once (two per CU), a multiple of its 8 XCDs.

@@ -82,7 +82,8 @@ int jh_op_gemm_ws(int epilogue, const void* x, size_t ldx, size_t rows, const vo
         a.w_ws = (const bf16_t*)w_packed;
         if (!gemm_ws_supported(epilogue, a))
             throw jh_error(1, "gemm: weight-stationary kernel needs packed W and K = 768 with N % 256 == 0, or K = "
-                              "1152 with N % 128 == 0 and the residual epilogue");
+                              "1152 with N % 128 == 0 and the residual epilogue, and rows of X and the output under "
+                              "2^28 bytes");
         if (!validate_gemm_args(epilogue, a)) return;
         launch_gemm_ws(epilogue, a, (hipStream_t)stream);
     });

@@ -82,6 +82,28 @@ def test_attention_item_limit(entry, window, ntiles, heads, refused):
     assert ("grid too large" in message) == refused, message
 
 
+@pytest.mark.skipif(os.path.exists("/dev/kfd"), reason="calls that pass the checks would be launched")
+@pytest.mark.parametrize("epi,k,ldx,ldo,refused", [
+    (abi.EPI_STORE_BF16, 768, 768, 256, False),
+    (abi.EPI_RESID_F32, 768, 768, (1 << 26) - 64, False),
+    (abi.EPI_RESID_F32, 768, 768, 1 << 26, True),
+    (abi.EPI_RESID_F32, 1152, 1152, 1 << 26, True),
+    (abi.EPI_BIAS_F32, 768, 768, 1 << 28, True),
+    (abi.EPI_STORE_BF16, 768, 768, (1 << 27) - 64, False),
+    (abi.EPI_GEGLU_BF16, 768, 768, 1 << 27, True),
+    (abi.EPI_STORE_BF16, 768, (1 << 27) - 64, 256, False),
+    (abi.EPI_STORE_BF16, 768, 1 << 27, 256, True),
+])
+def test_weight_stationary_stride_limit(epi, k, ldx, ldo, refused):
+    """The weight-stationary GEMM addresses 16 rows of X and of its output with 32-bit byte offsets: strides past that
+    are refused, and nothing below it.  Without a GPU, a call that passes the checks fails at the device."""
+    L, p = hip.lib(), 1 << 20
+    rc = L.jh_op_gemm_ws(epi, p, ldx, 17, p, 256, k, p, ldo, 0, p, p, p, p, 0, None)
+    message = L.jh_last_error().decode()
+    assert rc == (abi.JH_ERR_INVALID if refused else abi.JH_ERR_DEVICE), (rc, message)
+    assert ("weight-stationary" in message) == refused, message
+
+
 def test_create_rejects_bad_config_before_touching_device():
     cfg = synth.model_config("tiny")
     ws = abi.WeightSet(cfg, synth.make_weights(cfg, 0))
