@@ -1287,18 +1287,31 @@ int slab_waves(int epi, const GemmArgs& a) {
 //     7.1, 2500 22.3 / 12.2; N = 384 (672 tokens): 500 5.1 / 6.0, 700 13.8 / 6.1,
 //     4323 22.3 / 11.2.
 // W as it lies, row-major, takes 0.5 to 1.5 us longer to fetch, which moves the
-// lines: N = 2304, small-batch or tiled kernel against this one: 300 8.8 / 9.4,
-// 500 12.4 / 11.1, 2500 17.2 / 17.0, 3300 18.6 / 19.8, 4323 21.6 / 22.2, 6000
-// 30.8 / 27.5; K = 1152, N = 768: 7556 22.4 / 19.8, 16384 45.6 / 47.2.
+// lines (who passes it so: callers of jh_op_gemm_splitk, and the model for the marker rows).
+// Small-batch or tiled kernel against this one, bias epilogue unless named:
+//   N >= 1024, fewer than 128 tiles: N = 1024 800 tokens 9.9 / 8.3, 1900 11.2 / 9.6; N = 2304
+//     300 8.8 / 9.4, 500 12.4 / 9.3; N = 3072 300 10.1 / 8.6, 600 10.7 / 9.5;
+//   more: N = 2304 2500 17.2 / 17.0, 3300 18.6 / 19.8, 6000 24.7 / 25.2 (RoPE 30.9 / 27.7),
+//     7556 34.1 / 28.7, 32768 124 / 101; N = 1536 7556 21.9 / 22.1, 14000 38.8 / 34.8,
+//     49152 120 / 105; N = 1024 6000 14.4 / 15.4 and 16384 27.5 / 27.4, 65536 97 / 90;
+//     with the plain store N = 2304 6000 23.9 / 25.5, 7556 32.2 / 28.8, 40000 139 / 127, but
+//     49152 171 / 198, N = 1536 65536 153 / 179, N = 3072 40000 183 / 212;
+//   N < 1024: N = 768 2500 13.0 / 10.1, 7556 19.0 / 17.5, 131072 286 / 234; N = 256
+//     2500 11.9 / 8.2, 16384 15.8 / 15.5, 131072 107 / 80;
+//   K = 1152: N = 768 7556 23.2 / 20.1, 12000 39.4 / 26.6, 16384 45.6 / 47.2; N = 384 7556 17.6 /
+//     13.3, 24000 40.2 / 27.4; N = 128 4323 15.2 / 8.2, 32768 21.7 / 20.6, 65536 31.5 / 34.3.
 bool ws_takes(int epi, const GemmArgs& a) {
     if (!a.partial) return gemm_ws_supported(epi, a);
     if (!gemm_ws_shape(epi, a) || (a.w_ws && !gemm_ws_supported(epi, a)) || !narrow_strides(a)) return false;
     const long cus = resident_tiles() / 2, tiles = (long)((a.n + 127) / 128) * ((a.rows + 127) / 128);
     const long small = (long)(a.n / (a.k <= small_kmax<64>() ? 64 : 32)) * ((a.rows + SMALL_BT - 1) / SMALL_BT);
     if (a.w_ws) return a.n < 1024 || a.k > small_kmax<64>() ? small > cus : 4 * small > 5 * cus;
-    if (a.k > small_kmax<64>()) return small > cus && (long)a.rows * a.n < 12288L * 768;
+    const long out = (long)a.rows * a.n;
+    if (a.k > small_kmax<64>()) return small > cus && out < 12288L * 768 && a.rows <= 32768;
     if (a.n < 1024) return small > cus;
-    return tiles < 128 ? 2 * small > 3 * cus : a.rows >= 6000;
+    if (tiles < 128) return 2 * small > 3 * cus;
+    if (epi == JH_EPI_STORE_BF16) return out > 1L << 24 && out < 96L << 20;
+    return a.n >= 2048 ? a.rows >= 6000 : out > 1L << 24;
 }
 
 template <int EPI>
