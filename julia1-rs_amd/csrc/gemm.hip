@@ -1258,6 +1258,11 @@ bool narrow_strides(const GemmArgs& a) { return a.ldx <= 1L << 24 && a.ldo <= 1L
 //   N = 384: 933 4.0 / 5.3, 1500 4.9 / 6.8, 2500 5.8 / 6.5, 3000 6.8 / 6.5, 4323
 //     9.7 / 7.8, 7556 10.6 / 10.2, 16384 14.5 / 13.7, 65536 58.8 / 55.6: from the
 //     second round of the small-batch kernel's 64 x 32 tiles on (two per CU);
+//   N < 1024 with bf16 outputs, tiled kernel against this one: N = 384 4200 7.2 / 6.8, 9000 7.7 /
+//     8.4, 16384 9.6 / 10.6, 65536 29 / 25; N = 768 4200 7.7 / 8.5, 9000 10.4 / 11.5, 16384 15.8 /
+//     15.5, 65536 52 / 42; N = 256 16384 8.1 / 8.7, 65536 21 / 19: where the small-batch
+//     kernel still runs, and from 12 Mi outputs on (FP32 outputs: at all sizes, N = 768
+//     4200 9.7 / 9.5, 9000 15.1 / 14.3);
 //   N = 1152: 1200 6.7 / 7.0, 1500 8.3 / 6.8, 2500 9.5 / 9.8, 4323 12.2 / 12.7;
 //   N = 2304: 600 6.6 / 6.8, 700 7.2 / 6.7, 800 7.4 / 7.1, 1500 8.3 / 9.6: from one
 //     and a half rounds to the small-batch kernel's last size;
@@ -1268,7 +1273,8 @@ int slab_waves(int epi, const GemmArgs& a) {
     if (a.rows >= 16384 && a.n >= 1024 && a.n % 384 == 0) return 12;
     const long cus = resident_tiles() / 2, tiles = (long)((a.n + 127) / 128) * ((a.rows + 127) / 128);
     const long small = (long)(a.n / 64) * ((a.rows + SMALL_BT - 1) / SMALL_BT);
-    if (a.n < 1024) return small > 2 * cus ? 4 : 0;
+    const bool f32 = epi == JH_EPI_RESID_F32 || epi == JH_EPI_BIAS_F32;
+    if (a.n < 1024) return small > 2 * cus && (f32 || tiles < 128 || (long)a.rows * a.n >= 12L << 20) ? 4 : 0;
     return tiles < 128 && small > 3 * cus ? 4 : 0;
 }
 

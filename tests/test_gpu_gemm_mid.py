@@ -52,8 +52,9 @@ def _out(rows, width, epi, col, pad, seed):
 
 
 # (rows, n): the first ones each one row past (or at) the small-batch kernel's last size and the rule's end; then a
-# 128-row slab count that is no multiple of three, and 384-row slabs from 16384 rows on
-SLAB = [(2721, 384), (1345, 1152), (1792, 1152), (673, 2304), (4097, 256), (4323, 384), (16384, 1152), (16385, 2304),
+# 128-row slab count that is no multiple of three, 2^22 * 3 outputs (from where few columns of bf16 run here again), and
+# 384-row slabs from 16384 rows on
+SLAB = [(2721, 384), (1345, 1152), (1792, 1152), (673, 2304), (4097, 256), (4323, 384), (16384, 768), (16384, 1152), (16385, 2304),
         (20003, 1536)]
 
 
