@@ -398,7 +398,7 @@ __device__ __forceinline__ void attend(const AttnArgs& a, const AttnTile& tile, 
 // the split does not pay.  Measured (us, hidden 384, one row of 500 / 900 / 1500 /
 // 3928 keys): KS 1 10.0 / 15.1 / 22.0 / 50.4, KS 4 10.9 / 14.3 / 18.6 / 39.0; KS 2
 // at two items per CU: 8 rows of 900 keys 23.6 -> 23.9, 4 of 1500 31.4 -> 30.3.
-// Items of 32 or 64 queries: from kSplitRow keys on.  Below, they gain 2 us at 500 keys
+// Items of 64 queries: from kSplitRow keys on.  Below, they gain 2 us at 500 keys
 // (9.9 -> 8.0), 0.3 at 161 (6.5 -> 6.2, which the host's call hides) and 1.5 to 3.5% of a
 // request, but would make the sums of a short row, which most rows are, depend on
 // what else is in the launch.
@@ -458,20 +458,19 @@ void launch_items(const AttnArgs& a, hipStream_t s) {
     const bool win = a.window >= 0;
     // Few items leave SIMDs with one or two waves, or none.  The keys of each are
     // then split four (two) ways, and where the items are few for the CUs its
-    // queries over two or four workgroups too.  Only for rows of kSplitRow keys or more; the
+    // queries over two workgroups too.  Only for rows of kSplitRow keys or more; the
     // unsplit queries only over long rows (see kSplitKeys4), and not on window
     // layers, whose items have at most four or five key tiles.  Measured (us, one
     // row, hidden 384, full attention, 128-query items / four ways / and 64-query
     // workgroups): 933 keys 15.1 / 14.4 / 10.6, 1500 22.0 / 18.7 / 13.8, 2500 34.4 / 26.7 /
-    // 20.4; a whole request of 1200 tokens, 128-query items / 64 / 32: 1177 / 1121 / 1125.
+    // 20.4; a whole request of 1200 tokens, 128-query items / 64: 1177 / 1121.  (32-query
+    // workgroups of four waves at one item per eight CUs or less: within 0.1 us of these at 513
+    // to 1300 keys, 16.6 / 16.5 at 2000, and 0.4 us on a list of short rows.)
     // Where the caller does not say how long the rows are, a list too short to cover
     // one of kSplitRow queries runs unsplit: it would be run so anyway, and the larger
     // kernel's LDS and empty workgroups cost 0.1 us of 6.7 at 161 keys.
     const bool split = a.key_split && (a.longest ? a.longest >= kSplitRow : (long)a.ntiles * TQ >= kSplitRow);
-    if (split && 8 * items <= cus) {
-        if (win) JH_LAUNCH((attention_kernel<4, true, 4, TQ / 32>), grid(TQ / 32), dim3(256), 0, s, a);
-        else JH_LAUNCH((attention_kernel<4, false, 4, TQ / 32>), grid(TQ / 32), dim3(256), 0, s, a);
-    } else if (split && 2 * items <= cus) {
+    if (split && 2 * items <= cus) {
         if (win) JH_LAUNCH((attention_kernel<8, true, 4, TQ / 64>), grid(TQ / 64), dim3(512), 0, s, a);
         else JH_LAUNCH((attention_kernel<8, false, 4, TQ / 64>), grid(TQ / 64), dim3(512), 0, s, a);
     } else if (split && !win && items <= cus && (!a.longest || a.longest >= kSplitKeys4)) {

@@ -632,7 +632,7 @@ def test_attention_wide_items(heads, key_split, window):
 @pytest.mark.parametrize("heads,lens,key_split", [
     (2, [300, 257, 300, 190, 300], False),
     (2, [300, 257, 300, 190, 300], True),        # rows under 513 keys: as without the split
-    (2, [833, 900], True),                       # four ways, 32-query workgroups
+    (2, [833, 900], True),                       # four ways, 64-query workgroups
     (2, [900, 1025, 833, 1100, 1300], True),     # four ways, 64-query workgroups
     (5, [900, 1025, 833, 1100, 1300], True),     # four ways, 128-query items (full attention)
     (12, [1200, 1300, 1152], True),              # two ways (full attention)
@@ -675,9 +675,9 @@ def test_attention_rising_scores(heads, lens, key_split, window):
 @pytest.mark.parametrize("window", [-1, 2048])
 @pytest.mark.parametrize("heads,groups,group,pad", [
     (2, 1, 0, 0),    # keys not split: tiles 0 .. 3 of each row
-    (2, 4, 0, 0),    # four ways, 32-query workgroups: the first group's tiles
+    (2, 4, 0, 0),    # four ways, 64-query workgroups: the first group's tiles
     (2, 4, 3, 0),    # ... the last group's
-    (8, 4, 1, 0),    # four ways, 64-query workgroups
+    (8, 4, 1, 0),    # ... the second group's
     (16, 4, 2, 0),   # four ways, 128-query items (full attention)
     (16, 2, 1, 12),  # two ways (full attention, 1152 keys or more)
 ])
@@ -762,14 +762,14 @@ def test_attention_full_length_8192(window):
 @pytest.mark.parametrize("rate", [0.0, 0.4])
 @pytest.mark.parametrize("window", [-1, 64, 8])
 @pytest.mark.parametrize("heads,lens,wide", [
-    (2, [513, 700, 30], False),            # at most 32 items: 32-query workgroups, keys split four ways from 513 keys on
-    (2, [831, 832, 300, 960, 1], False),   # at most 128: 64-query workgroups
+    (2, [513, 700, 30], False),            # at most 128 items: 64-query workgroups, keys split four ways from 513 keys on
+    (2, [831, 832, 300, 960, 1], False),
     (6, [831, 832, 833, 1], False),        # at most one 128-query item per CU: split from 832 keys on
     (12, [1151, 1152, 1153, 130], False),  # up to two per CU: two ways from 1152 on
     (12, [1407, 1300], True),              # 144 tiles of 256 queries: the eight-wave kernel, unsplit (full attention)
     (6, [1407, 1300], True),               # 72: as two 128-query workgroups each, split four ways (full attention)
     (32, [1407, 1300], True),              # 384: as two 128-query workgroups each, unsplit
-    (2, [900, 257], True),                 # ... and as eight of 32 queries
+    (2, [900, 257], True),                 # ... and as four of 64 queries
 ])
 def test_attention_key_split(heads, lens, wide, window, rate):
     """Few work items: groups of waves take every second or fourth key tile and merge their running maxima, sums and
