@@ -63,27 +63,6 @@ __device__ inline i32x4 make_rsrc(const void* base, uint64_t bytes) {
                  (int)(uint32_t)(bytes < 0xffffffffull ? bytes : 0xffffffffull), 0x00020000};
 }
 
-// Work item of workgroup b of G, item numbers in contiguous runs per XCD (workgroup
-// b runs on XCD b % 8).
-__device__ inline int xcd_run(int b, int G) {
-    const int xcd = b & 7, q8 = G >> 3, r8 = G & 7;
-    return xcd * q8 + (xcd < r8 ? xcd : r8) + (b >> 3);
-}
-
-// Item (slab f of nF, token range r of nR) of a workgroup of the GEMMs that keep W
-// resident.  An XCD's L2 holds what its own workgroups fetch: with items in token
-// order it fetches its eighth of X and all of W, in slab order its eighth of W and
-// all of X.  Slab order is taken where W is the larger, N > tokens.  Measured (us,
-// token / slab order, W not in L2): K = 768 packed, N = 3072 382 tokens 10.0 / 8.6,
-// N = 2304 500 tokens 9.4 / 8.7, 1000 tokens 10.4 / 9.7, row-major N = 768 700 tokens 8.2 / 8.0;
-// K = 1152, N = 768 500 tokens 7.4 / 7.0; K = 384, N = 2304 700 tokens 7.6 / 6.4.
-__device__ inline void xcd_item(int b, int nF, int nR, bool slab_order, int& f, int& r) {
-    const int u = xcd_run(b, nF * nR);
-    const int d = slab_order ? nR : nF, hi = u / d, lo = u - hi * d;
-    f = slab_order ? hi : lo;
-    r = slab_order ? lo : hi;
-}
-
 // v plus the same value of lane l ^ STEP, for a butterfly that takes its steps from
 // 32 down to 1, the order of sums that the wavefronts of this library have always
 // had: half-wave and 16-lane swaps, then DPP within 16 lanes (a rotation by 8, by 4

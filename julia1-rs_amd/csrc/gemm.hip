@@ -964,9 +964,17 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(GemmArgs a) {
     __shared__ __align__(1024) bf16_t smem[LDS];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nF = a.n / BF;
-    // (Plain order: xcd_item's runs took a request of 161 tokens from 673 to 684 us,
-    // Wo of it from 2.86 to 2.97; single launches went both ways by up to 5%.)
-    const int f0 = (int)(blockIdx.x % nF) * BF, t0 = (int)(blockIdx.x / nF) * BT;
+    // Tile of the workgroup, features varying fastest.  Where tokens are the more, an
+    // XCD (workgroup b runs on XCD b % 8) takes a contiguous run of tiles, as the row
+    // kernels deal their rows: one row of 1300 tokens at hidden 384 1129 -> 1119 us.
+    // Runs in either order for fewer tokens cost: 161 tokens, by features 670 -> 684 us,
+    // at hidden 768 by tokens 808 -> 850.
+    int u = (int)blockIdx.x;
+    if (a.rows >= a.n) {
+        const int G = gridDim.x, xcd = u & 7, q8 = G >> 3, r8 = G & 7;
+        u = xcd * q8 + (xcd < r8 ? xcd : r8) + (u >> 3);
+    }
+    const int f0 = u % nF * BF, t0 = u / nF * BT;
     const int nseg = CSEG ? CSEG : a.k / 64;  // 128-byte row segments
     bf16_t* const sW = smem;                   // segment g: rows [0, BF) at sW + g*BF*64
     bf16_t* const sX = smem + nseg * BF * 64;  // segment g: rows [0, BT) at sX + g*BT*64

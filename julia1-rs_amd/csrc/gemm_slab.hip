@@ -79,8 +79,12 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 4
 
     const int lane = threadIdx.x & 63, tk = lane & 15, kg = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    int f, r;  // slab and token range
-    xcd_item((int)blockIdx.x, nF, R, a.n > a.rows, f, r);
+    // Workgroup -> (token range r, slab f): consecutive u share r, and an XCD
+    // (workgroup b runs on XCD b % 8) takes a contiguous run of u.
+    const int G = gridDim.x, bid = blockIdx.x;
+    const int xcd = bid & 7, q8 = G >> 3, r8 = G & 7;
+    const int u = xcd * q8 + (xcd < r8 ? xcd : r8) + (bid >> 3);
+    const int r = u / nF, f = u - r * nF;
     const int u0 = (int)((long)r * nU / R), nu = (int)((long)(r + 1) * nU / R) - u0;  // this range's units
     if (nu <= 0) return;
 
