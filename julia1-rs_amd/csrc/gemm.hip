@@ -1303,8 +1303,10 @@ int slab_waves(int epi, const GemmArgs& a) {
 // W as it lies, row-major, takes 0.5 to 1.5 us longer to fetch, which moves the
 // lines (who passes it so: callers of jh_op_gemm_splitk, and the model for the marker rows).
 // Small-batch or tiled kernel against this one, bias epilogue unless named:
-//   N >= 1024, fewer than 128 tiles: N = 1024 800 tokens 9.9 / 8.3, 1900 11.2 / 9.6; N = 2304
-//     300 8.8 / 9.4, 500 12.4 / 9.3; N = 3072 300 10.1 / 8.6, 600 10.7 / 9.5;
+//   N >= 1024, fewer than 128 tiles: from the small-batch kernel's third round on. Two rounds
+//     N = 1024 800 tokens 8.0 / 8.6, N = 1536 600 8.1 / 8.9, N = 2304 400 8.1 / 9.5, N = 3072 300 8.1 /
+//     10.4; three 1200 11.2 / 9.4, 800 11.2 / 9.8, 500 11.2 / 10.4, 382 11.2 / 11.2; four 1900
+//     14.4 / 9.8, 1200 14.5 / 10.0, 800 14.4 / 10.7, 600 14.6 / 11.5;
 //   more: N = 2304 2500 17.2 / 17.0, 3300 18.6 / 19.8, 6000 24.7 / 25.2 (RoPE 30.9 / 27.7),
 //     7556 34.1 / 28.7, 32768 124 / 101; N = 1536 7556 21.9 / 22.1, 14000 38.8 / 34.8,
 //     49152 120 / 105; N = 1024 6000 14.4 / 15.4 and 16384 27.5 / 27.4, 65536 97 / 90;
@@ -1323,7 +1325,7 @@ bool ws_takes(int epi, const GemmArgs& a) {
     const long out = (long)a.rows * a.n;
     if (a.k > small_kmax<64>()) return small > cus && out < 12288L * 768 && a.rows <= 32768;
     if (a.n < 1024) return small > cus;
-    if (tiles < 128) return 2 * small > 3 * cus;
+    if (tiles < 128) return small > 2 * cus;
     if (epi == JH_EPI_STORE_BF16) return out > 1L << 24 && out < 96L << 20;
     return a.n >= 2048 ? a.rows >= 6000 : out > 1L << 24;
 }

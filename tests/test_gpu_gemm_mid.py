@@ -85,7 +85,7 @@ def test_slab_against_64_bits(rows, n, epi):
 
 @pytest.mark.parametrize("rows,n,k,epi", [
     (673, 768, 768, abi.EPI_RESID_F32), (2687, 768, 768, abi.EPI_BIAS_F32), (2049, 256, 768, abi.EPI_STORE_BF16),
-    (2053, 256, 768, abi.EPI_BIAS_F32), (353, 2304, 768, abi.EPI_ROPE_BF16), (896, 2304, 768, abi.EPI_GEGLU_BF16),
+    (2053, 256, 768, abi.EPI_BIAS_F32), (449, 2304, 768, abi.EPI_ROPE_BF16), (896, 2304, 768, abi.EPI_GEGLU_BF16),
     (6001, 2304, 768, abi.EPI_ROPE_BF16), (6000, 2304, 768, abi.EPI_GEGLU_BF16), (382, 3072, 768, abi.EPI_BIAS_RELU_BF16),
     (700, 768, 768, abi.EPI_BIAS_BF16), (673, 384, 1152, abi.EPI_RESID_F32), (2049, 128, 1152, abi.EPI_RESID_F32),
     (321, 768, 1152, abi.EPI_RESID_F32), (4323, 384, 1152, abi.EPI_RESID_F32)])
