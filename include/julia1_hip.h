@@ -186,19 +186,23 @@ int jh_collect(jh_model* model, uint64_t ticket, float* scores, size_t markers);
 int jh_set_graph(jh_model* model, int enabled);
 
 /*
- * Small-batch GEMM paths (1 = on, default; 0 = off).  When a GEMM's output has
- * too few 128 x 128 tiles to occupy the GPU (small batches, marker rows), K is
- * split: over the four waves of one workgroup (one launch, K <= 768) or into
- * chunks whose FP32 partial sums a second kernel reduces (the residual GEMMs,
- * with the residual add and LayerNorm in that kernel).  Attention over few
- * rows likewise splits the keys of a query over groups of waves.
- * Either way the partial
- * sums are added in a fixed order, so results are deterministic, but a row's
- * FP32 summation order then depends on the batch's token count.  Off, every output element is accumulated in the same
- * order whatever the batch, so a row's logits are invariant to what else is
- * batched with it (to FP32 round-off of the bf16 activations, <= 1e-4), at
- * the cost of small-batch latency.  No reference counterpart (cuBLAS picks
- * its own split per shape).
+ * Kernels chosen by the size of the batch (1 = on, default; 0 = off).  On:
+ *  - GEMMs with too few 128 x 128 tiles to occupy the GPU (small batches,
+ *    marker rows) split K, over the four waves of one workgroup (one launch,
+ *    K <= 768) or into chunks whose FP32 partial sums a second kernel reduces
+ *    (the residual GEMMs, with the residual add and LayerNorm in that kernel);
+ *  - larger ones at K = 384, 768 and 1152 go to the kernels that keep W in
+ *    registers as soon as those are faster, at some hundreds of tokens, and at
+ *    K = 384 again from 16384 tokens;
+ *  - attention splits the keys of rows of 513 tokens or more over groups of
+ *    waves where the batch has few work items.
+ * Sums are added in a fixed order, so results are deterministic, but a row's
+ * FP32 order then depends on the batch's token count: a row's logits move by
+ * up to about 2e-3 between batches (hidden 768; 6e-4 at hidden 384).  Off,
+ * every output element is accumulated in the same order whatever the batch, so
+ * a row's logits are invariant to what else is batched with it (to FP32
+ * round-off of the bf16 activations, <= 1e-4), at the cost of small-batch
+ * latency.  No reference counterpart (cuBLAS picks its own split per shape).
  */
 int jh_set_splitk(jh_model* model, int enabled);
 

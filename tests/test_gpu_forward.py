@@ -291,6 +291,44 @@ def test_hidden_384_shape(shape):
         check_gates(s)
 
 
+@pytest.mark.parametrize("splitk", [False, True])
+@pytest.mark.parametrize("shape", ["julia1", "modernbert-base"])
+def test_rows_with_split_keys(shape, splitk):
+    """Rows of 513 tokens and more, whose keys a small batch splits over groups of waves, at both hidden sizes: alone
+    against the oracle, and against themselves beside a shorter row, in a batch of rows around the splits' limits and
+    among enough other rows that nothing is split.  With split-K off a row's scores do not depend on the batch (1e-4,
+    as test_batching_invariance); with it on, the FP32 order of its attention and GEMM sums does, which bf16
+    activations carry through 22 layers: up to 6.4e-4 at hidden 384 and 1.9e-3 at 768 over six inputs of eleven lengths
+    each (5.8e-4 and 1.9e-3 with attention unsplit), so within the 2e-3 that split-K keeps to."""
+    cfg = synth.model_config(shape)
+    ws = abi.WeightSet(cfg, synth.make_weights(cfg, seed=5))
+    gpu = hip.HipModel(ws)
+    gpu.set_splitk(splitk)
+    r = np.random.default_rng(513)
+    lens = [513, 600, 832, 1700, 2500, 161, 500]
+    rows = [(r.integers(0, cfg.vocab, n, dtype=np.uint32), [1, n // 3, n // 2, n - 1], i % 3)
+            for i, n in enumerate(lens)]
+    fill = [(r.integers(0, cfg.vocab, 700, dtype=np.uint32), [3, 400], 0) for _ in range(20)]
+    batch = abi.Batch.from_items
+    alone = [gpu.forward(batch([row])) for row in rows]
+    if splitk:
+        orc = oracle.OracleModel(ws, threads=8)
+        for row, got in zip(rows[:5], alone):
+            check_gates(parity(batch([row]), got, orc.forward(batch([row]))))
+    limit, worst = 2e-3 if splitk else 1e-4, 0.0
+    for mates in ([rows[5]], rows, rows + fill):
+        for i, row in enumerate(rows):
+            if mates is rows or len(mates) > len(rows):
+                b, at = batch(mates), i
+            else:
+                b, at = batch([row] + mates), 0
+            got = b.split_scores(gpu.forward(b))[at]
+            worst = max(worst, float(np.abs(got - alone[i]).max()))
+    print(shape, splitk, "alone against batched", worst)
+    assert worst <= limit, worst
+    gpu.close()
+
+
 @pytest.mark.parametrize("tokens,fused", [(1024, True), (1025, False), (1280, False)])
 def test_fused_small_layers_only_on_the_small_kernel(tokens, fused):
     """The LayerNorms move into the small-batch GEMMs' prologues only where all four projections of a layer run as
