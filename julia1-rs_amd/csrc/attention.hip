@@ -453,7 +453,7 @@ double halves_cost(long items, long cus) {
 // The 128-query items of the list's tiles, TQ / 128 to a tile.
 template <int TQ>
 void launch_items(const AttnArgs& a, hipStream_t s) {
-    const long cus = gemm_resident_tiles() / 2, items = (long)a.ntiles * a.heads * (TQ / 128);
+    const long items = (long)a.ntiles * a.heads * (TQ / 128);
     auto grid = [&](int sub) { return dim3((unsigned)((long)a.ntiles * a.heads * sub)); };
     const bool win = a.window >= 0;
     // Few items leave SIMDs with one or two waves, or none.  The keys of each are
@@ -470,6 +470,7 @@ void launch_items(const AttnArgs& a, hipStream_t s) {
     // one of kSplitRow queries runs unsplit: it would be run so anyway, and the larger
     // kernel's LDS and empty workgroups cost 0.1 us of 6.7 at 161 keys.
     const bool split = a.key_split && (a.longest ? a.longest >= kSplitRow : (long)a.ntiles * TQ >= kSplitRow);
+    const long cus = split ? gemm_resident_tiles() / 2 : 0;  // (asks the runtime for the device)
     if (split && 2 * items <= cus) {
         if (win) JH_LAUNCH((attention_kernel<8, true, 4, TQ / 64>), grid(TQ / 64), dim3(512), 0, s, a);
         else JH_LAUNCH((attention_kernel<8, false, 4, TQ / 64>), grid(TQ / 64), dim3(512), 0, s, a);
@@ -499,9 +500,12 @@ void launch_attention(const AttnArgs& a, hipStream_t s) {
     const long items = (long)a.ntiles * a.heads, most = 0x7fffffffL;
     if (items > most || (a.waves == 8 && a.window >= 0 && 2 * items > most))
         throw jh_error(1, "attention: grid too large");
-    const long cus = gemm_resident_tiles() / 2;
+    auto halves = [&] {
+        const long cus = gemm_resident_tiles() / 2;
+        return 2 * items <= most && halves_cost(items, cus) < wide_cost(items, cus);
+    };
     if (a.waves == 4) launch_items<128>(a, s);
-    else if (a.window >= 0 || (2 * items <= most && halves_cost(items, cus) < wide_cost(items, cus))) launch_items<256>(a, s);
+    else if (a.window >= 0 || halves()) launch_items<256>(a, s);
     else JH_LAUNCH((attention_kernel<8, false>), dim3((unsigned)items), dim3(512), 0, s, a);
     HIP_CHECK(hipGetLastError());
 }

@@ -318,8 +318,10 @@ def op_attention(q, ldq, k, v, ldkv, out, ldo, tiles, heads, window, scale=0.125
     """q/k/v/out torch bf16 tensors (base pointers of the first row/col); tiles torch int32 [n, 5] of at most
     128 queries each, or 256 with wide=True (eight-wave work items, jh_op_attention_wide); key_split=False keeps
     each query's keys in one wave (jh_op_attention_unsplit)."""
-    fn = lib().jh_op_attention_wide if wide else lib().jh_op_attention
-    last = (stream,)
     if not key_split:
-        fn, last = lib().jh_op_attention_unsplit, (1 if wide else 0, stream)
-    check(fn(_dp(q), ldq, _dp(k), _dp(v), ldkv, _dp(out), ldo, _dp(tiles), tiles.shape[0], heads, window, scale, *last))
+        check(lib().jh_op_attention_unsplit(_dp(q), ldq, _dp(k), _dp(v), ldkv, _dp(out), ldo, _dp(tiles), tiles.shape[0],
+                                            heads, window, scale, 1 if wide else 0, stream))
+        return
+    fn = lib().jh_op_attention_wide if wide else lib().jh_op_attention
+    check(fn(_dp(q), ldq, _dp(k), _dp(v), ldkv, _dp(out), ldo, _dp(tiles), tiles.shape[0], heads, window, scale,
+             stream))
