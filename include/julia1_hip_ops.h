@@ -109,8 +109,8 @@ int jh_op_gemm_ln(int epilogue, const float* xf, size_t ldx, size_t rows, const 
  * the fragment order jh_op_pack_ws writes.  Shapes: K == 768 with N % 256 ==
  * 0 (256-row slabs, every epilogue), or K == 1152 with N % 128 == 0 and
  * JH_EPI_RESID_F32 only (128-row slabs, K split between partner waves whose
- * two half sums are added lower half first); no row gather.  Other arguments
- * as jh_op_gemm.  The same bf16 products as jh_op_gemm, summed in FP32 in K
+ * two half sums are added lower half first); no row gather; rows of X and of
+ * the output under 2^28 bytes.  Other arguments as jh_op_gemm.  The same bf16 products as jh_op_gemm, summed in FP32 in K
  * order in steps of 32 (jh_op_gemm: 16), so outputs agree to FP32 rounding.
  * jh_forward uses it for the K = 768 GEMMs and the MLP-out projection
  * (K = intermediate = 1152) outside the small-batch path.  Replaces cuBLAS
